@@ -84,19 +84,21 @@ def read_variant_list():
 
 def parse_resource_remarks(text):
     """Maps (BM,BN,BK,WM,WN,S,G,persistent) -> resource dict from -Rpass-analysis
-    output."""
+    output; a row's kernel with non-temporal stores has "nt" behind its key."""
     out = {}
     cur = None
     name_re = re.compile(r"Function Name: (\S+)")
     tmpl_re = re.compile(
-        r"gemmMfma(PingPong|Persistent)?KernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E")
+        r"gemmMfma(PingPong|Persistent)?KernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E(?:Lb([01])E)?")
     field_re = re.compile(r"remark:\s+([A-Za-z][A-Za-z /\[\]]*?):\s*(\S+)")
     for line in text.splitlines():
         m = name_re.search(line)
         if m:
             t = tmpl_re.search(m.group(1))
-            cur = (tuple(int(x) for x in t.groups()[1:]) + (1 if t.group(1) == "Persistent" else 0,)
+            cur = (tuple(int(x) for x in t.groups()[1:8]) + (1 if t.group(1) == "Persistent" else 0,)
                    if t else None)
+            if cur is not None and t.group(9) == "1":
+                cur += ("nt",)  # the non-temporal form of a row: gated, not in the table
             if cur is not None:
                 out[cur] = {}
             continue
@@ -137,7 +139,7 @@ def build_gemm(gate=True):
     missing = [v for v in variants if v not in res]
     if missing:
         raise SystemExit("no resource remarks for variants %s" % missing)
-    spilling = [v for v in variants
+    spilling = [v for v in res
                 if res[v]["scratch"] != 0 or res[v]["vgpr_spill"] != 0 or res[v]["sgpr_spill"] != 0]
     print("  %d variants, %d spilling" % (len(variants), len(spilling)))
     for v in spilling:

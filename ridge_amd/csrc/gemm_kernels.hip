@@ -67,19 +67,29 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
     return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int S, int G>
-hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
+template <int BM, int BN, int BK, int WM, int WN, int S, int G, bool NT>
+void enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
     using T = ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>;
     const dim3 grid((unsigned)((M / BM) * (N / BN)));
     const dim3 block(T::kThreads);
     if constexpr (usesPingPong(T::kWaves, S)) {
-        hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G>), grid, block, 0, stream,
-                           static_cast<const _Float16*>(A), static_cast<const _Float16*>(B),
-                           static_cast<_Float16*>(C), M, N, K);
+        hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>), grid, block, 0, stream, A, B,
+                           C, M, N, K);
     } else {
-        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G>), grid, block, 0, stream,
-                           static_cast<const _Float16*>(A), static_cast<const _Float16*>(B),
-                           static_cast<_Float16*>(C), M, N, K);
+        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), grid, block, 0, stream, A, B, C, M,
+                           N, K);
+    }
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int S, int G>
+hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
+    const auto* a = static_cast<const _Float16*>(A);
+    const auto* b = static_cast<const _Float16*>(B);
+    auto* c = static_cast<_Float16*>(C);
+    if ((size_t)M * N * 2 > ridge::kNonTemporalBytes) {
+        enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
+    } else {
+        enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);
     }
     return hipGetLastError();
 }

@@ -261,7 +261,7 @@ __device__ __forceinline__ void staticFor(F&& f) {
 // and the 16-byte reads (8 lanes along a row) are both conflict-free. Up to 8
 // read-backs are in flight before their stores issue. The global stores are
 // not waited for; NT marks them non-temporal (streamed past the caches), which
-// lifts a C-bound kernel's write rate when C is not re-read soon.
+// lifts the write rate of a C that the caches would not keep anyway.
 template <int TM, int TN, int WN, int EPI, bool NT>
 __device__ __forceinline__ void storeStaged(const float4_t (&acc)[TM][TN], RIDGE_LDS_AS char* region,
                                             _Float16* cWave, int N, int lane) {
@@ -316,6 +316,18 @@ __device__ __forceinline__ void storeStaged(const float4_t (&acc)[TM][TN], RIDGE
         if (passC.value + 1 < TM / EPI) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     });
 }
+
+// A C of more than this is stored non-temporally by the uniform and ping-pong
+// kernels (NT; a template argument, because the compiler merged the two stores of
+// a run-time choice and dropped the hint). Written through the caches such a C
+// evicts the A and B panels from the L2s that the running workgroups share, and
+// leaves a write-back behind the kernel: 8192 x 8192 x 1024 in 256x256x32 tiles
+// 136.0 -> 117.4 us, x 512 97.3 -> 73.3. A smaller C stays cached, because the
+// kernel that reads it next finds it there: at 3072 x 3072 (18.9 MB)
+// non-temporal stores made the GEMM itself 10% faster, but it and a GEMM that
+// follows on C 14% slower together; at 5120 x 5120 (52 MB) 0 and 1% slower, at
+// 6144 x 6144 (75 MB) 1% and 2% faster.
+constexpr size_t kNonTemporalBytes = (size_t)64 << 20;
 
 // Per-workgroup state and the operations both schedules are built from: the
 // output tile, the direct-to-LDS refill of a stage, the fragment reads of a
@@ -468,16 +480,14 @@ struct GemmBlock {
             }
     }
 
-    // Epilogue through LDS (storeStaged below). Regions are per wave, so the
+    // Epilogue through LDS (storeStaged above). Regions are per wave, so the
     // only cross-wave hazard is the ring they overlay: every wave must be past
-    // its last ring read (a barrier) before the call. Waves whose whole tile does
-    // not fit the ring at once make several passes of kEpiTiles 16-row tile-rows.
-    static constexpr int epiTiles() {
-        int p = TM;
-        while (p > 1 && (TM % p != 0 || T::kWaves * 16 * p * WN * 2 > T::kLdsBytes)) --p;
-        return p;
-    }
-    static constexpr int kEpiTiles = epiTiles();
+    // its last ring read (a barrier) before the call. One 16-row tile-row per
+    // pass: the stores of a pass leave while the next one is converted, and
+    // against passes of as many rows as the ring holds it measured 0.3-1.5%
+    // faster on every row (256x256x64 s2 at 4096 x 4096 x 1024 with
+    // non-temporal stores 33.4 -> 32.2 us).
+    static constexpr int kEpiTiles = 1;
     static constexpr int kEpiRegionBytes = 16 * kEpiTiles * WN * 2;
     static_assert(T::kWaves * kEpiRegionBytes <= T::kLdsBytes, "epilogue regions must fit the ring");
 
@@ -486,11 +496,10 @@ struct GemmBlock {
         return C + (size_t)(blockRow + waveM * WM) * N + blockCol + waveN * WN;
     }
 
-    // Regular (cached) stores: these kernels are timed, like the reference's,
-    // on operands re-used across launches, where C stays in the MALL.
+    template <bool NT>
     __device__ __forceinline__ void store(_Float16* C, int N) const {
         RIDGE_LDS_AS char* region = (RIDGE_LDS_AS char*)(const_cast<char*>(lds)) + wave * kEpiRegionBytes;
-        storeStaged<TM, TN, WN, kEpiTiles, false>(acc, region, waveC(C, N), N, lane);
+        storeStaged<TM, TN, WN, kEpiTiles, NT>(acc, region, waveC(C, N), N, lane);
     }
 };
 
@@ -517,7 +526,7 @@ __device__ __forceinline__ void interleaveHint() {
 // its reads of tile kt, the freed stage is refilled with tile kt+STAGES and
 // tile kt+1's first fragments are read while tile kt's last MFMAs run.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                     _Float16* __restrict__ C, int M, int N, int K) {
@@ -614,7 +623,7 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
     for (; kt0 < numK; kt0 += U) pass(kt0, std::false_type{});
     // Every wave is past its last ring read before the epilogue reuses LDS.
     barrierLds();
-    blk.store(C, N);
+    blk.template store<NT>(C, N);
 }
 
 // ---------------------------------------------------------------------------
@@ -644,7 +653,7 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
 //    waits there until at most tiles t+2 .. t+STAGES-1 of its own loads are
 //    outstanding.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                             _Float16* __restrict__ C, int M, int N, int K) {
@@ -727,7 +736,7 @@ void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __re
     } else {
         runGroup(std::integral_constant<int, 1>{});
     }
-    blk.store(C, N);
+    blk.template store<NT>(C, N);
 }
 
 // ---------------------------------------------------------------------------

@@ -414,9 +414,10 @@ def cmd_run(args):
 # ---------------------------------------------------------------------------
 
 # Kernel names as rocprofv3 reports them: Itanium-mangled, each int template
-# argument as Li<n>E (gemmMfmaKernelILi64ELi64E...), or demangled (<64, 64, ...>).
+# argument as Li<n>E (gemmMfmaKernelILi64ELi64E...), or demangled (<64, 64, ...>);
+# a bool argument (non-temporal stores) may follow the seven ints.
 _GEMM_NAME = re.compile(r"gemmMfma(?:PingPong|Persistent)?Kernel(?:I" + r"Li(\d+)E" * 7 + r"|<" +
-                        r",".join([r"\s*(\d+)"] * 7) + r"\s*>)")
+                        r",".join([r"\s*(\d+)"] * 7) + r"\s*(?:,\s*(?:true|false)\s*)?>)")
 
 
 def _template_args(name):
