@@ -46,17 +46,32 @@ int residentSlots(const void* kernel, int threads, std::atomic<int>& cache) {
 
 constexpr int kMaxDevices = 64;
 
+// Resident workgroups of a kernel on the current device; 0 with *err set when the
+// device cannot be asked.
+struct SlotCache {
+    std::atomic<int> slots[kMaxDevices];
+    int of(const void* kernel, int threads, hipError_t* err) {
+        int dev = 0;
+        *err = hipGetDevice(&dev);
+        if (*err != hipSuccess) return 0;
+        if (dev < 0 || dev >= kMaxDevices) {
+            *err = hipErrorInvalidDevice;
+            return 0;
+        }
+        const int n = residentSlots(kernel, threads, slots[dev]);
+        if (n <= 0) *err = hipErrorInvalidConfiguration;
+        return n > 0 ? n : 0;
+    }
+};
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
 hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
     using P = ridge::PersistentTraits<BM, BN, BK, WM, WN, S, G>;
-    static std::atomic<int> slots[kMaxDevices];
-    int dev = 0;
-    hipError_t err = hipGetDevice(&dev);
-    if (err != hipSuccess) return err;
-    if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-    const void* kernel = reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>);
-    const int resident = residentSlots(kernel, P::kThreads, slots[dev]);
-    if (resident <= 0) return hipErrorInvalidConfiguration;
+    static SlotCache cache;
+    hipError_t err;
+    const int resident = cache.of(
+        reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), P::kThreads, &err);
+    if (resident <= 0) return err;
     // Every workgroup must own at least one tile (the kernel's tile count per
     // workgroup assumes it).
     const int tiles = (M / BM) * (N / BN);
@@ -67,18 +82,49 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
     return hipGetLastError();
 }
 
+// Parts per output tile of the last round of a ping-pong grid: `rem` tiles on
+// `slots` CUs, one workgroup each. Whole, they hold rem CUs for the time of a tile
+// while the others idle. The line is where the parts still fit one round; a second
+// round of parts costs more than the whole tile. 256x256x32 s3, whole -> cut:
+//   quarters   5888 x 5888 x 1664 (2 rounds and 17 tiles)  112.8 -> 97.2 us
+//              4352 x 4096 x 1024 (1 round and 16)          46.7 -> 36.2
+//              4352 x 4096 x 256                            19.7 -> 16.3
+//              2048^3 (64 tiles)                            35.0 -> 18.8
+//   halves     2560^3 (100 tiles)                           44.2 -> 34.6
+//              4864 x 4864 x 1024 (1 round and 105)         48.4 -> 45.0
+//   K no multiple of the quarters' 64: halves, 5888 x 5888 x 1632 107.6 -> 100.3
+// 256x128x64 s3 (halves are the same 128 x 128 parts): 2304 x 4096 x 2048 (1 round
+// and 32) 50.2 -> 42.8, 2048^3 (128 tiles) 23.2 -> 19.6.
+int tailParts(int rem, int slots, int K, int most) {
+    if (rem == 0) return 1;
+    if (most >= 4 && K % 64 == 0 && 4 * rem <= slots) return 4;
+    if (most >= 2 && 2 * rem <= slots) return 2;
+    return 1;
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G, bool NT>
-void enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
+hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
     using T = ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>;
-    const dim3 grid((unsigned)((M / BM) * (N / BN)));
+    const int tiles = (M / BM) * (N / BN);
     const dim3 block(T::kThreads);
     if constexpr (usesPingPong(T::kWaves, S)) {
+        static SlotCache cache;
+        hipError_t err;
+        const int slots = cache.of(
+            reinterpret_cast<const void*>(&ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>), T::kThreads,
+            &err);
+        // A device that does not say its slots runs every tile whole.
+        const int rem = slots > 0 ? tiles % slots : 0;
+        const int parts = tailParts(rem, slots, K, ridge::TailTiles<BM, BN, BK>::kParts);
+        const int whole = parts > 1 ? tiles - rem : tiles;
+        const dim3 grid((unsigned)(whole + (tiles - whole) * parts));
         hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>), grid, block, 0, stream, A, B,
-                           C, M, N, K);
+                           C, M, N, K, whole, parts);
     } else {
-        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), grid, block, 0, stream, A, B, C, M,
-                           N, K);
+        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
+                           stream, A, B, C, M, N, K);
     }
+    return hipGetLastError();
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
@@ -86,12 +132,9 @@ hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, in
     const auto* a = static_cast<const _Float16*>(A);
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
-    if ((size_t)M * N * 2 > ridge::kNonTemporalBytes) {
-        enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
-    } else {
-        enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);
-    }
-    return hipGetLastError();
+    if ((size_t)M * N * 2 > ridge::kNonTemporalBytes)
+        return enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
+    return enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);
 }
 
 struct Entry {

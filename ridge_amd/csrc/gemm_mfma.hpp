@@ -198,6 +198,7 @@ __device__ __forceinline__ void phaseBarrier() {
 
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
 struct GemmTraits {
+    static constexpr int kStages = STAGES;
     static constexpr int kWavesM = BM / WM;
     static constexpr int kWavesN = BN / WN;
     static constexpr int kWaves = kWavesM * kWavesN;
@@ -345,8 +346,6 @@ struct GemmBlock {
     uint32_t ldsBase;     // its LDS byte address (scalar)
     int lane, wave, waveM, waveN;
     int blockRow, blockCol;
-    const _Float16* baseA;
-    const _Float16* baseB;
     const char* gA;       // A + blockRow * K (bytes), scalar
     const char* gB;       // B + blockCol (bytes), scalar
     size_t tileStrideB;   // bytes between K tiles of B: BK * N * 2
@@ -358,8 +357,8 @@ struct GemmBlock {
     int numKTiles;        // K / BK
     int kStart = 0;       // first K tile of the loop of issueTile<true>, which wraps
 
-    __device__ __forceinline__ GemmBlock(const char* ldsArray, const _Float16* A, const _Float16* B, int M,
-                                         int N, int K) {
+    __device__ __forceinline__ GemmBlock(const char* ldsArray, const _Float16* A, const _Float16* B, int row,
+                                         int col, int N, int K) {
         lds = ldsArray;
         ldsBase = ldsAddress(ldsArray);
         lane = threadIdx.x % kWaveSize;
@@ -368,9 +367,10 @@ struct GemmBlock {
         waveM = wave / T::kWavesN;
         waveN = wave % T::kWavesN;
 
-        baseA = A;
-        baseB = B;
-        setTile(xcdRemap(blockIdx.x, gridDim.x), M, N, K);
+        blockRow = row;
+        blockCol = col;
+        gA = reinterpret_cast<const char*>(A + (size_t)row * K);
+        gB = reinterpret_cast<const char*>(B + col);
         tileStrideB = (size_t)BK * N * 2;
         numKTiles = K / BK;
         // Wave instruction j fills physical chunks [64 j, 64 j + 64) of a tile;
@@ -413,14 +413,6 @@ struct GemmBlock {
             for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[tm][tn][e] = 0.0f;
-    }
-
-    // The output tile of logical launch id `pid` (after the XCD remap) in the
-    // GroupM launch order (reference gemm-mma.cuh:158-178), and its operand bases.
-    __device__ __forceinline__ void setTile(int pid, int M, int N, int K) {
-        tileOf<BM, BN, GROUPM>(pid, M, N, blockRow, blockCol);
-        gA = reinterpret_cast<const char*>(baseA + (size_t)blockRow * K);
-        gB = reinterpret_cast<const char*>(baseB + blockCol);
     }
 
     // Refills LDS stage `stage` with K tile kTile (this wave's share). No vector
@@ -526,40 +518,19 @@ __device__ __forceinline__ void interleaveHint() {
 // its reads of tile kt, the freed stage is refilled with tile kt+STAGES and
 // tile kt+1's first fragments are read while tile kt's last MFMAs run.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
-void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                    _Float16* __restrict__ C, int M, int N, int K) {
-    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
-    using Blk = GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+template <bool STAGGER, bool STEADY, typename Blk>
+__device__ __forceinline__ void uniformLoop(Blk& blk, int numK) {
+    using T = typename Blk::T;
+    constexpr int STAGES = T::kStages;
     constexpr int TM = T::kTilesM;
     constexpr int TN = T::kTilesN;
     constexpr int KS = T::kSteps;
     constexpr int L = T::kLoadsPerTile;
 
-    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
-    Blk blk(lds, A, B, M, N, K);
-    const int numK = K / BK;
-    // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
-    // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
-    // Cold, when the first touch of every K slice comes from HBM, workgroups in
-    // lockstep all request the same K slice of their panels at once (A's slice
-    // strided by a row); staggered, they request different slices. Measured at
-    // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
-    // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
-    // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
-    // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
-    // long K loops, which gained nothing. Only the summation order of the K tiles
-    // changes.
-    constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
-    if constexpr (kStagger) {
-        if (numK <= 32) blk.kStart = (blk.blockRow / BM + blk.blockCol / BN) % numK;
-    }
-
     // Prologue: every stage filled; a tile that does not exist is not issued,
     // and the waits count only issued loads (near the end of K they drain fully).
     staticFor<STAGES>([&](auto sC) {
-        if (sC.value < numK) blk.template issueTile<kStagger>(sC.value, sC.value);
+        if (sC.value < numK) blk.template issueTile<STAGGER>(sC.value, sC.value);
     });
     if (numK >= STAGES) {
         waitVmcnt<(STAGES - 1) * L>();
@@ -605,7 +576,7 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
                         // This wave's reads of tile kt are complete (lgkmcnt(0)) and
                         // every wave arrived: stage s is free and tile kt+1 visible.
                         barrierLds();
-                        if (steady || kt + STAGES < numK) blk.template issueTile<kStagger>(kt + STAGES, s);
+                        if (steady || kt + STAGES < numK) blk.template issueTile<STAGGER>(kt + STAGES, s);
                         blk.template readFrags<sNext>(0, fa[cur ^ 1], fb[cur ^ 1]);
                     }
                     blk.mfmaStep(fa[cur], fb[cur]);
@@ -614,15 +585,44 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
             }
         });
     };
-    // The 8-wave rows (two stages, 256 registers per lane) keep the general form
-    // only: the second copy of the loop made them spill.
     int kt0 = 0;
-    if constexpr (T::kWaves <= 4) {
+    if constexpr (STEADY) {
         for (; kt0 + U - 1 + STAGES < numK; kt0 += U) pass(kt0, std::true_type{});
     }
     for (; kt0 < numK; kt0 += U) pass(kt0, std::false_type{});
     // Every wave is past its last ring read before the epilogue reuses LDS.
     barrierLds();
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
+void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
+                    _Float16* __restrict__ C, int M, int N, int K) {
+    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
+    int row, col;
+    tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, gridDim.x), M, N, row, col);
+    GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
+    const int numK = K / BK;
+    // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
+    // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
+    // Cold, when the first touch of every K slice comes from HBM, workgroups in
+    // lockstep all request the same K slice of their panels at once (A's slice
+    // strided by a row); staggered, they request different slices. Measured at
+    // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
+    // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
+    // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
+    // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
+    // long K loops, which gained nothing. Only the summation order of the K tiles
+    // changes.
+    constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
+    if constexpr (kStagger) {
+        if (numK <= 32) blk.kStart = (blk.blockRow / BM + blk.blockCol / BN) % numK;
+    }
+
+    // The 8-wave rows (two stages, 256 registers per lane) keep the general form
+    // of the loop only: the second copy made them spill.
+    uniformLoop<kStagger, (T::kWaves <= 4)>(blk, numK);
     blk.template store<NT>(C, N);
 }
 
@@ -653,23 +653,17 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
 //    waits there until at most tiles t+2 .. t+STAGES-1 of its own loads are
 //    outstanding.
 // ---------------------------------------------------------------------------
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
-void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                            _Float16* __restrict__ C, int M, int N, int K) {
-    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
-    using Blk = GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+template <typename Blk>
+__device__ __forceinline__ void pingPongLoop(Blk& blk, int numK) {
+    using T = typename Blk::T;
     static_assert(T::kWaves == 8, "ping-pong pairs two groups of four wavefronts");
-    static_assert(STAGES >= 3, "ping-pong refills one tile ahead of two in flight");
+    static_assert(T::kStages >= 3, "ping-pong refills one tile ahead of two in flight");
+    constexpr int STAGES = T::kStages;
     constexpr int TM = T::kTilesM;
     constexpr int TN = T::kTilesN;
     constexpr int KS = T::kSteps;
     constexpr int L = T::kLoadsPerTile;
-
-    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
-    Blk blk(lds, A, B, M, N, K);
     const int group = blk.wave / 4;
-    const int numK = K / BK;
 
     staticFor<STAGES - 1>([&](auto sC) {
         if (sC.value < numK) blk.issueTile(sC.value, sC.value);
@@ -736,7 +730,86 @@ void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __re
     } else {
         runGroup(std::integral_constant<int, 1>{});
     }
-    blk.template store<NT>(C, N);
+}
+
+// The parts into which the ping-pong kernel cuts the output tiles of a last,
+// partial round (tailParts in gemm_kernels.hip says when). A part is a workgroup of
+// the same launch, on the row's LDS, with a block shape and loop of its own. Every
+// output still sums its products in K order, so C is the whole tile's bit for bit.
+template <int BM, int BN, int BK>
+struct TailTiles {
+    static constexpr int kParts = 1;      // the most parts of one tile
+    static constexpr int kLdsBytes = 0;
+};
+
+// 128 x 128 parts: BK = 64 and eight 32 x 64 wave tiles on the uniform loop, so that
+// the two wavefronts of a SIMD hide each other's barriers and LDS latency. At 2048^3
+// (one part per CU) 18.8 us, of which about 5 are launch, first fetch and epilogue;
+// 64 x 32 wave tiles 19.1, BK = 32 19.9, the ping-pong loop 20.6 (its memory phase
+// outlasts its 256-cycle matrix phase), deeper rings within 1%.
+struct TailQuarter {
+    using Blk = GemmBlock<128, 128, 64, 32, 64, 3, 1>;
+    template <bool NT>
+    static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
+                                               int row, int col, int N, int K) {
+        Blk blk(lds, A, B, row, col, N, K);
+        uniformLoop<false, true>(blk, K / 64);
+        blk.template store<NT>(C, N);
+    }
+};
+
+template <>
+struct TailTiles<256, 256, 32> {
+    static constexpr int kParts = 4;
+    using Half = GemmBlock<128, 256, 32, 64, 64, 3, 1>;
+    static constexpr int kLdsBytes = TailQuarter::Blk::T::kLdsBytes > Half::T::kLdsBytes
+                                         ? TailQuarter::Blk::T::kLdsBytes
+                                         : Half::T::kLdsBytes;
+    template <bool NT>
+    static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
+                                               int row, int col, int part, int parts, int N, int K) {
+        if (parts == 4) {
+            TailQuarter::run<NT>(lds, A, B, C, row + 128 * (part / 2), col + 128 * (part % 2), N, K);
+        } else {
+            Half blk(lds, A, B, row + 128 * part, col, N, K);
+            pingPongLoop(blk, K / 32);
+            blk.template store<NT>(C, N);
+        }
+    }
+};
+
+template <>
+struct TailTiles<256, 128, 64> {
+    static constexpr int kParts = 2;
+    static constexpr int kLdsBytes = TailQuarter::Blk::T::kLdsBytes;
+    template <bool NT>
+    static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
+                                               int row, int col, int part, int parts, int N, int K) {
+        TailQuarter::run<NT>(lds, A, B, C, row + 128 * part, col, N, K);
+    }
+};
+
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
+void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
+                            _Float16* __restrict__ C, int M, int N, int K, int wholeTiles, int parts) {
+    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+    using Tail = TailTiles<BM, BN, BK>;
+    static_assert(Tail::kLdsBytes <= T::kLdsBytes, "the parts of a tile use the row's ring");
+    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
+    int row, col;
+    if ((int)blockIdx.x < wholeTiles) {
+        tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, wholeTiles), M, N, row, col);
+        GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
+        pingPongLoop(blk, K / BK);
+        blk.template store<NT>(C, N);
+    } else if constexpr (Tail::kParts > 1) {
+        // The tail tiles are the last of the launch order; the parts of one tile
+        // are neighbours and share an XCD.
+        const int id = xcdRemap(blockIdx.x - wholeTiles, gridDim.x - wholeTiles);
+        tileOf<BM, BN, GROUPM>(wholeTiles + id / parts, M, N, row, col);
+        Tail::template run<NT>(lds, A, B, C, row, col, id % parts, parts, N, K);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -915,7 +988,7 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
         return;
     }
 
-    Blk blk(lds, A, B, M, N, K);
+    Blk blk(lds, A, B, 0, 0, N, K);
     RIDGE_LDS_AS char* region = (RIDGE_LDS_AS char*)(lds) + T::kLdsBytes + wave * P::kRegionBytes;
     barrierLds();  // B_0
     half8_t fa[2][TM];
@@ -951,7 +1024,7 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
                     interleaveHint<TM, TN>();
                 }
                 if (++kt == numK) {
-                    blk.setTile(self + tile * grid, M, N, K);
+                    tileOf<BM, BN, GROUPM>(self + tile * grid, M, N, blk.blockRow, blk.blockCol);
                     // Non-temporal: measured +21% cold and +1% warm at 8192^2 x 128.
                     storeStaged<TM, TN, WN, P::kEpiTiles, true>(blk.acc, region, blk.waveC(C, N), N, lane);
 #pragma unroll

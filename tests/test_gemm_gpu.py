@@ -300,6 +300,23 @@ def test_c_at_the_non_temporal_threshold_bit_exact(M, N, K):
         assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
 
 
+# Output tiles of 256 x 256 around the tail rule's edges on 256 CUs: up to a
+# quarter round is cut into quarter tiles (K a multiple of 64), up to half a round
+# into half tiles; alone and behind a whole round.
+@pytest.mark.parametrize("tiles_m,tiles_n,K", [
+    (1, 1, 64), (1, 1, 96), (8, 8, 448), (8, 8, 96), (13, 5, 64), (13, 5, 480), (16, 8, 192), (43, 3, 64),
+    (257, 1, 64), (257, 1, 32), (20, 16, 256), (107, 3, 128), (24, 16, 64), (77, 5, 64)])
+def test_ping_pong_tail_tiles_bit_exact(tiles_m, tiles_n, K):
+    M, N = 256 * tiles_m, 256 * tiles_n
+    Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + 3 * N + 7 * K)
+    A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
+    for v in G.variants():
+        if v.schedule != 1 or not v.divides(M, N, K):
+            continue
+        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
+        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+
+
 def _persistent_edge_shapes(v):
     """Shapes that drive the persistent schedule's control flow to its edges."""
     BM, BN, BK, S = v.BM, v.BN, v.BK, v.stages
