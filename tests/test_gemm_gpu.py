@@ -56,6 +56,21 @@ def test_device_fills_match_oracle_bit_exact():
         assert np.array_equal(_bits(t), O.uniform_fill_f16(n, seed)), seed
 
 
+# One chunk is 2048 elements where dst is 16-byte aligned and 256 elsewhere; 2048
+# workgroups take a chunk each before the grid stride.
+@pytest.mark.parametrize("offset", [0, 1, 7, 8])
+@pytest.mark.parametrize("n", [1, 7, 9, 2047, 2049, 256 * 2048 + 3, 2048 * 2048 * 2 + 2051])
+def test_device_fills_at_chunk_edges_and_any_alignment(n, offset):
+    t = torch.full((n + 16,), 7.0, dtype=torch.float16, device=DEV)
+    for fill, want in ((G.fill_uniform, O.uniform_fill_f16), (G.fill_lcg, O.lcg_fill_f16)):
+        t.fill_(7.0)
+        fill(t[offset:offset + n], 0xFFFFFFF3)
+        got = _bits(t)
+        assert np.array_equal(got[offset:offset + n], want(n, 0xFFFFFFF3))
+        outside = np.concatenate([got[:offset], got[offset + n:]])
+        assert np.all(outside == np.float16(7.0).view(np.uint16)), "wrote outside its range"
+
+
 @pytest.mark.parametrize("M,N,K", REFERENCE_SHAPES)
 def test_reference_shapes_all_dividing_variants(M, N, K):
     print("shape %dx%dx%d" % (M, N, K), flush=True)

@@ -214,3 +214,12 @@ def test_fp16_output_bound_closed_forms():
     assert O.passes_fp16(ref + two_ulp, ref, absprod, 1)[2] > 1.0
     g = O.fp16_output_bound(np.zeros((1, 1)), np.array([[4.0]]), 1024)
     assert g[0, 0] == pytest.approx((1 + 2.0 ** -11) * 1.001 * 1024 * 2.0 ** -24 * 4.0 + 2.0 ** -25)
+
+
+def test_lcg_value_by_reciprocal_equals_the_quotient_for_every_draw():
+    """fill.hip multiplies by the float reciprocal of 32767 (product and difference
+    rounded separately): the same half as the division for all 32768 draws."""
+    x = np.arange(32768).astype(np.float32)
+    quotient = (x / np.float32(32767.0) - np.float32(0.5)).astype(np.float16)
+    product = (x * (np.float32(1.0) / np.float32(32767.0)) - np.float32(0.5)).astype(np.float16)
+    assert np.array_equal(quotient.view(np.uint16), product.view(np.uint16))
