@@ -179,6 +179,10 @@ def _ptr(x):
 def _stream_handle(stream):
     if stream is None:
         import torch
+        if torch.cuda.is_initialized():
+            # The same handle without building a Stream object (2.8 -> 0.5 us, of a
+            # launch that costs 4).
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
@@ -265,8 +269,11 @@ def gemm(A, B, index=0, out=None, stream=None):
     N = B.shape[1]
     C = out if out is not None else torch.empty((M, N), dtype=torch.float16, device=A.device)
     # The library launches on the current device; make it the operands' one.
-    with torch.cuda.device(A.device):
+    if torch._C._cuda_getDevice() == A.device.index:
         rc = launch(index, A, B, C, M, N, K, stream)
+    else:
+        with torch.cuda.device(A.device):
+            rc = launch(index, A, B, C, M, N, K, stream)
     if rc != HIP_SUCCESS:
         raise RidgeGemmError("ridge_gemm_launch(variant %d, %dx%dx%d) returned hipError %d" % (index, M, N, K, rc))
     return C
