@@ -44,6 +44,11 @@ HIP_FLAGS = [
     "-I" + INCLUDE, "-I" + CSRC,
 ]
 
+# Kernel arguments of the library's kernels arrive in scalar registers instead of by
+# a load that every workgroup waits for: 0.22 us off each launch (1024^3 5.91 -> 5.69
+# us). Not for the calibration benches, whose constants were measured without it.
+LIB_HIP_FLAGS = HIP_FLAGS + ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
+
 _RESOURCE_KEYS = {
     "VGPRs": "vgprs",
     "AGPRs": "agprs",
@@ -133,7 +138,7 @@ def build_gemm(gate=True):
     os.makedirs(LIB, exist_ok=True)
     variants = read_variant_list()
     kobj = os.path.join(BUILD, "gemm_kernels.o")
-    remarks = _run([HIPCC] + HIP_FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-c",
+    remarks = _run([HIPCC] + LIB_HIP_FLAGS + ["-Rpass-analysis=kernel-resource-usage", "-c",
                                           os.path.join(CSRC, "gemm_kernels.hip"), "-o", kobj], capture=True)
     res = parse_resource_remarks(remarks)
     missing = [v for v in variants if v not in res]
@@ -153,7 +158,7 @@ def build_gemm(gate=True):
     for src in ("fill.hip", "blaslt.cpp"):
         o = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
         lang = ["-x", "hip"] if src.endswith(".hip") else []
-        _run([HIPCC] + HIP_FLAGS + lang + ["-c", os.path.join(CSRC, src), "-o", o])
+        _run([HIPCC] + (LIB_HIP_FLAGS if lang else HIP_FLAGS) + lang + ["-c", os.path.join(CSRC, src), "-o", o])
         objs.append(o)
     o = os.path.join(BUILD, "gemm_resources.gen.o")
     _run([CXX, "-O2", "-fPIC", "-std=c++17", "-I" + INCLUDE, "-I" + CSRC, "-c", gen, "-o", o])

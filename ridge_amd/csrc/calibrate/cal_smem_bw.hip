@@ -325,7 +325,9 @@ __global__ __launch_bounds__(((BM / WM) * (BN / WN) + ridge::kPersistentLoaders)
     // One column of tiles, one per workgroup: the block only forms its LDS
     // fragment offsets here and reads no global memory; mode 3 writes C.
     const int rowsC = BM * (int)gridDim.x * (Mode == 3 ? kEpiSlots : 1);
-    Blk blk(lds, src, src, rowsC, BN, BK * G);
+    Blk blk(lds, src, src, BM * (int)blockIdx.x, 0, BN, BK * G);
+    const ridge::TileOrder order = ridge::tileOrder<BM, BN, 8>(rowsC, BN);
+    (void)order;
     RIDGE_LDS_AS char* region = (RIDGE_LDS_AS char*)(lds) + T::kLdsBytes + wave * P::kRegionBytes;
     (void)region;
     // The kernel's own tile cursor: a K-tile count compared with K / BK, and the
@@ -368,7 +370,8 @@ __global__ __launch_bounds__(((BM / WM) * (BN / WN) + ridge::kPersistentLoaders)
                 }
                 if constexpr (Mode == 3) {
                     if (++kt == tileK) {
-                        blk.setTile((int)blockIdx.x * kEpiSlots + (tile % kEpiSlots), rowsC, BN, BK * G);
+                        ridge::tileOf<BM, BN, 8>((int)blockIdx.x * kEpiSlots + (tile % kEpiSlots), rowsC, BN, order,
+                                                 blk.blockRow, blk.blockCol);
                         ridge::storeStaged<TM, TN, WN, P::kEpiTiles, true>(blk.acc, region, blk.waveC(C, BN), BN,
                                                                            lane);
 #pragma unroll
@@ -416,7 +419,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void pingPongRowSkeleto
     __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
     // One column of tiles, one per workgroup: the block forms its LDS fragment
     // offsets; its loads are `issue` below, from the four-tile source.
-    Blk blk(lds, src, src, BM * (int)gridDim.x, BN, BK * G);
+    Blk blk(lds, src, src, BM * (int)blockIdx.x, 0, BN, BK * G);
     const int wave = blk.wave;
     const int lane = blk.lane;
     const int group = wave / 4;
@@ -520,7 +523,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void uniformRowSkeleton
     constexpr int L = T::kLoadsPerTile;
     constexpr int kTileBytes = T::kBytesA + T::kBytesB;
     __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
-    Blk blk(lds, src, src, BM * (int)gridDim.x, BN, BK * G);
+    Blk blk(lds, src, src, BM * (int)blockIdx.x, 0, BN, BK * G);
     const int wave = blk.wave;
     const int lane = blk.lane;
     uint32_t offA[T::kPerWaveA], offB[T::kPerWaveB];

@@ -75,10 +75,12 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
     // Every workgroup must own at least one tile (the kernel's tile count per
     // workgroup assumes it).
     const int tiles = (M / BM) * (N / BN);
-    const dim3 grid((unsigned)(tiles < resident ? tiles : resident));
-    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), grid, dim3(P::kThreads), 0,
-                       stream, static_cast<const _Float16*>(A), static_cast<const _Float16*>(B),
-                       static_cast<_Float16*>(C), M, N, K);
+    const int grid = tiles < resident ? tiles : resident;
+    const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
+    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), dim3((unsigned)grid),
+                       dim3(P::kThreads), 0, stream, static_cast<const _Float16*>(A),
+                       static_cast<const _Float16*>(B), static_cast<_Float16*>(C), M, N, K, order.group,
+                       order.lastRows, ridge::reciprocalOf(K / BK), grid, tiles / grid, tiles % grid);
     return hipGetLastError();
 }
 
@@ -107,6 +109,7 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
     using T = ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>;
     const int tiles = (M / BM) * (N / BN);
     const dim3 block(T::kThreads);
+    const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
     if constexpr (usesPingPong(T::kWaves, S)) {
         static SlotCache cache;
         hipError_t err;
@@ -117,12 +120,13 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
         const int rem = slots > 0 ? tiles % slots : 0;
         const int parts = tailParts(rem, slots, K, ridge::TailTiles<BM, BN, BK>::kParts);
         const int whole = parts > 1 ? tiles - rem : tiles;
-        const dim3 grid((unsigned)(whole + (tiles - whole) * parts));
-        hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>), grid, block, 0, stream, A, B,
-                           C, M, N, K, whole, parts);
+        const int partTiles = (tiles - whole) * parts;
+        hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>),
+                           dim3((unsigned)(whole + partTiles)), block, 0, stream, A, B, C, M, N, K, order.group,
+                           order.lastRows, whole, partTiles, parts);
     } else {
         hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
-                           stream, A, B, C, M, N, K);
+                           stream, A, B, C, M, N, K, order.group, order.lastRows, ridge::reciprocalOf(K / BK));
     }
     return hipGetLastError();
 }

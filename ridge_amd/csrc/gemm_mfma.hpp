@@ -129,18 +129,52 @@ __device__ __forceinline__ int xcdRemap(int pid, int n) {
     return x * q + (x < r ? x : r) + pid / kXcds;
 }
 
+// Division by a launch's constants without a divide: q = floor(n * floor(2^32 / d) /
+// 2^32) is the quotient or one less for every n < 2^32, and one step corrects it. The
+// compiler's 32-bit divide is about 40 dependent vector and scalar instructions, and
+// two or three of them stood between a workgroup's start and its first load.
+__host__ __device__ inline uint32_t reciprocalOf(uint32_t d) {
+    return d <= 1 ? 0xffffffffu : (uint32_t)(0x100000000ull / d);
+}
+
+struct DivMod {
+    uint32_t quot, rem;
+};
+
+__host__ __device__ __forceinline__ DivMod divide(uint32_t n, uint32_t d, uint32_t reciprocal) {
+    uint32_t q = (uint32_t)(((uint64_t)n * reciprocal) >> 32);
+    uint32_t r = n - q * d;
+    if (r >= d) {
+        ++q;
+        r -= d;
+    }
+    return {q, r};
+}
+
 // GroupM launch order: logical id pid -> (row, column) of the output tile's
 // first element. Groups of GROUPM tile rows are walked column by column, so
-// consecutive ids share B column panels and a group shares A row panels.
+// consecutive ids share B column panels and a group shares A row panels. The
+// reciprocals, made on the host (tileOrder), are those of a group's tile count and
+// of the last group's rows.
+struct TileOrder {
+    uint32_t group, lastRows;
+};
+
 template <int BM, int BN, int GROUPM>
-__device__ __forceinline__ void tileOf(int pid, int M, int N, int& row, int& col) {
-    const int numPidM = M / BM;
-    const int numPidN = N / BN;
-    const int pidInGroup = pid % (GROUPM * numPidN);
-    const int firstPidM = (pid / (GROUPM * numPidN)) * GROUPM;
-    const int groupRows = min(numPidM - firstPidM, GROUPM);
-    row = (firstPidM + pidInGroup % groupRows) * BM;
-    col = (pidInGroup / groupRows) * BN;
+__host__ __device__ inline TileOrder tileOrder(int M, int N) {
+    return {reciprocalOf((uint32_t)GROUPM * (uint32_t)(N / BN)), reciprocalOf((uint32_t)(M / BM) % GROUPM)};
+}
+
+template <int BM, int BN, int GROUPM>
+__host__ __device__ __forceinline__ void tileOf(int pid, int M, int N, TileOrder order, int& row, int& col) {
+    static_assert((GROUPM & (GROUPM - 1)) == 0, "whole groups divide by shifts");
+    const uint32_t numPidM = M / BM;
+    const DivMod group = divide((uint32_t)pid, (uint32_t)GROUPM * (uint32_t)(N / BN), order.group);
+    const uint32_t firstPidM = group.quot * GROUPM;
+    DivMod in = {group.rem / GROUPM, group.rem % GROUPM};
+    if (numPidM - firstPidM < GROUPM) in = divide(group.rem, numPidM - firstPidM, order.lastRows);
+    row = (int)(firstPidM + in.rem) * BM;
+    col = (int)in.quot * BN;
 }
 
 // Direct-to-LDS 16-byte load: lane t of the wave writes LDS bytes
@@ -597,11 +631,13 @@ __device__ __forceinline__ void uniformLoop(Blk& blk, int numK) {
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                    _Float16* __restrict__ C, int M, int N, int K) {
+                    _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
+                    uint32_t lastRowsReciprocal, uint32_t numKReciprocal) {
     using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
     int row, col;
-    tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, gridDim.x), M, N, row, col);
+    const int tiles = (M / BM) * (N / BN);  // = gridDim.x, which would be a load
+    tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
     GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
     const int numK = K / BK;
     // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
@@ -617,7 +653,7 @@ void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__
     // changes.
     constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
     if constexpr (kStagger) {
-        if (numK <= 32) blk.kStart = (blk.blockRow / BM + blk.blockCol / BN) % numK;
+        if (numK <= 32) blk.kStart = (int)divide((uint32_t)(row / BM + col / BN), numK, numKReciprocal).rem;
     }
 
     // The 8-wave rows (two stages, 256 registers per lane) keep the general form
@@ -792,23 +828,26 @@ struct TailTiles<256, 128, 64> {
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                            _Float16* __restrict__ C, int M, int N, int K, int wholeTiles, int parts) {
+                            _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
+                            uint32_t lastRowsReciprocal, int wholeTiles, int partTiles, int parts) {
     using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using Tail = TailTiles<BM, BN, BK>;
     static_assert(Tail::kLdsBytes <= T::kLdsBytes, "the parts of a tile use the row's ring");
     __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
     int row, col;
     if ((int)blockIdx.x < wholeTiles) {
-        tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, wholeTiles), M, N, row, col);
+        tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, wholeTiles), M, N, {groupReciprocal, lastRowsReciprocal}, row,
+                               col);
         GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
         pingPongLoop(blk, K / BK);
         blk.template store<NT>(C, N);
     } else if constexpr (Tail::kParts > 1) {
         // The tail tiles are the last of the launch order; the parts of one tile
         // are neighbours and share an XCD.
-        const int id = xcdRemap(blockIdx.x - wholeTiles, gridDim.x - wholeTiles);
-        tileOf<BM, BN, GROUPM>(wholeTiles + id / parts, M, N, row, col);
-        Tail::template run<NT>(lds, A, B, C, row, col, id % parts, parts, N, K);
+        const int id = xcdRemap(blockIdx.x - wholeTiles, partTiles);
+        const int shift = parts / 2;  // parts is 2 or 4
+        tileOf<BM, BN, GROUPM>(wholeTiles + (id >> shift), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
+        Tail::template run<NT>(lds, A, B, C, row, col, id & (parts - 1), parts, N, K);
     }
 }
 
@@ -868,7 +907,9 @@ struct PersistentTraits {
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
 __global__ __launch_bounds__(((BM / WM) * (BN / WN) + kPersistentLoaders) * kWaveSize)
 void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                              _Float16* __restrict__ C, int M, int N, int K) {
+                              _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
+                              uint32_t lastRowsReciprocal, uint32_t numKReciprocal, int grid, int tilesEach,
+                              int tilesMore) {
     using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using P = PersistentTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using Blk = GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM>;
@@ -880,12 +921,12 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
     __shared__ __attribute__((aligned(1024))) char lds[P::kLdsBytes];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
-    const int grid = gridDim.x;
     const int self = xcdRemap(blockIdx.x, grid);
-    const int numTiles = (M / BM) * (N / BN);
+    const TileOrder order = {groupReciprocal, lastRowsReciprocal};
     const int numK = K / BK;
-    // The launcher makes grid <= numTiles, so every workgroup has a tile.
-    const int G = ((numTiles - self + grid - 1) / grid) * numK;
+    // The launcher makes grid <= the tile count, so every workgroup has a tile:
+    // tilesEach, and one more for the first tilesMore workgroups.
+    const int G = (tilesEach + (self < tilesMore ? 1 : 0)) * numK;
 
     if (wave >= T::kWaves) {
         // Loader wave l issues wave instructions l, l + kLoaders, ... of each
@@ -913,11 +954,11 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
         // a row panel keep one order and share A in L2. Only the summation order
         // of the K tiles changes.
         int curTile = 0, curK = 0, row, col;
-        tileOf<BM, BN, GROUPM>(self, M, N, row, col);
+        tileOf<BM, BN, GROUPM>(self, M, N, order, row, col);
         const size_t strideB = (size_t)BK * N * 2;
         const char* srcA = reinterpret_cast<const char*>(A + (size_t)row * K);
         const char* srcB = reinterpret_cast<const char*>(B + col);
-        int kIdx = (row / BM) % numK;
+        int kIdx = (int)divide((uint32_t)(row / BM), numK, numKReciprocal).rem;
         uint32_t kOffA = (uint32_t)kIdx * BK * 2;
         size_t kOffB = (size_t)kIdx * strideB;
         auto issueNext = [&](int stage) {
@@ -945,10 +986,10 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
             }
             if (++curK == numK && ++curTile * numK < G) {
                 curK = 0;
-                tileOf<BM, BN, GROUPM>(self + curTile * grid, M, N, row, col);
+                tileOf<BM, BN, GROUPM>(self + curTile * grid, M, N, order, row, col);
                 srcA = reinterpret_cast<const char*>(A + (size_t)row * K);
                 srcB = reinterpret_cast<const char*>(B + col);
-                kIdx = (row / BM) % numK;
+                kIdx = (int)divide((uint32_t)(row / BM), numK, numKReciprocal).rem;
                 kOffA = (uint32_t)kIdx * BK * 2;
                 kOffB = (size_t)kIdx * strideB;
             }
@@ -1024,7 +1065,7 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
                     interleaveHint<TM, TN>();
                 }
                 if (++kt == numK) {
-                    tileOf<BM, BN, GROUPM>(self + tile * grid, M, N, blk.blockRow, blk.blockCol);
+                    tileOf<BM, BN, GROUPM>(self + tile * grid, M, N, order, blk.blockRow, blk.blockCol);
                     // Non-temporal: measured +21% cold and +1% warm at 8192^2 x 128.
                     storeStaged<TM, TN, WN, P::kEpiTiles, true>(blk.acc, region, blk.waveC(C, N), N, lane);
 #pragma unroll

@@ -332,6 +332,20 @@ def test_ping_pong_tail_tiles_bit_exact(tiles_m, tiles_n, K):
         assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
 
 
+@pytest.mark.parametrize("tiles_m", [1, 2, 3, 7, 8, 9, 17, 31])
+@pytest.mark.parametrize("tiles_n", [1, 3, 13])
+def test_launch_order_with_ragged_groups_bit_exact(tiles_m, tiles_n):
+    """Grids whose last launch-order group has every number of tile rows: the order
+    divides by reciprocals made on the host. C starts as NaN, so a tile that no
+    workgroup computes shows."""
+    M, N, K = 256 * tiles_m, 256 * tiles_n, 128
+    Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + 5 * N)
+    A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
+    for v in G.variants():
+        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
+        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+
+
 def _persistent_edge_shapes(v):
     """Shapes that drive the persistent schedule's control flow to its edges."""
     BM, BN, BK, S = v.BM, v.BN, v.BK, v.stages
