@@ -104,6 +104,19 @@ int tailParts(int rem, int slots, int K, int most) {
     return 1;
 }
 
+// Workgroups per step of the first round's phased start, 0 for none: grids of three
+// whole rounds and more whose K loop is short enough that the shared drains of C count
+// for more than the last step's 7168 cycles. 256x256x32 s3, together -> phased (two
+// devices): 8192 x 8192 x 256 47.6 -> 45.4, 58.0 -> 46.3 us; x 1024 114.4 -> 112.6,
+// 117.8 -> 111.7; x 2048 198.7 -> 197.6, 203.4 -> 201.0; x 3072 304.0 -> 303.3; 9728 x
+// 6400 x 768 88.3 -> 86.0, 93.0 -> 85.2; 15104 x 15104 x 512 219.5 -> 216.5, 232.9 ->
+// 224.4; 256x128x64 s3 at 8192 x 4096 x 512 41.6 -> 39.8, 49.8 -> 46.6. Two rounds
+// gained up to 20% on one device and lost up to 2% on another (8192 x 4096 x 512 40.2
+// -> 36.9, 34.8 -> 34.9; 6144 x 6144 x 512 41.5 -> 42.3).
+int phaseWidth(int wholeTiles, int slots, int K) {
+    return slots >= ridge::kPhases && wholeTiles / slots >= 3 && K <= 2048 ? slots / ridge::kPhases : 0;
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G, bool NT>
 hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
     using T = ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>;
@@ -123,7 +136,8 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
         const int partTiles = (tiles - whole) * parts;
         hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>),
                            dim3((unsigned)(whole + partTiles)), block, 0, stream, A, B, C, M, N, K, order.group,
-                           order.lastRows, whole, partTiles, parts);
+                           order.lastRows, whole, partTiles,
+                           parts | phaseWidth(whole, slots, K) << 8);
     } else {
         hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
                            stream, A, B, C, M, N, K, order.group, order.lastRows, ridge::reciprocalOf(K / BK));

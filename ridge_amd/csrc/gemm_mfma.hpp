@@ -768,6 +768,8 @@ __device__ __forceinline__ void pingPongLoop(Blk& blk, int numK) {
     }
 }
 
+constexpr int kPhases = 8;   // steps of the phased start
+
 // The parts into which the ping-pong kernel cuts the output tiles of a last,
 // partial round (tailParts in gemm_kernels.hip says when). A part is a workgroup of
 // the same launch, on the row's LDS, with a block shape and loop of its own. Every
@@ -829,12 +831,23 @@ template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool N
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                             _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
-                            uint32_t lastRowsReciprocal, int wholeTiles, int partTiles, int parts) {
+                            uint32_t lastRowsReciprocal, int wholeTiles, int partTiles, int partsAndPhase) {
     using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using Tail = TailTiles<BM, BN, BK>;
     static_assert(Tail::kLdsBytes <= T::kLdsBytes, "the parts of a tile use the row's ring");
     __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
     int row, col;
+    // Two counts in one argument: fourteen preloaded registers hold the arguments.
+    const int parts = partsAndPhase & 0xff;
+    const int phaseWidth = partsAndPhase >> 8;
+    // Phased start (phaseWidth in gemm_kernels.hip says when): the workgroups of
+    // the first round begin 1024 cycles apart in kPhases steps. Started together,
+    // the CUs reach the end of their tiles together in every round and share the
+    // memory's write rate while the matrix pipes idle; apart, one group's C drains
+    // under the others' K loops.
+    if ((int)blockIdx.x < kPhases * phaseWidth) {
+        for (int i = (int)blockIdx.x / phaseWidth; i > 0; --i) __builtin_amdgcn_s_sleep(16);
+    }
     if ((int)blockIdx.x < wholeTiles) {
         tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, wholeTiles), M, N, {groupReciprocal, lastRowsReciprocal}, row,
                                col);
