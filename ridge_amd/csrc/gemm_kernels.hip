@@ -90,16 +90,23 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
 // round of parts costs more than the whole tile. 256x256x32 s3, whole -> cut:
 //   quarters   5888 x 5888 x 1664 (2 rounds and 17 tiles)  112.8 -> 97.2 us
 //              4352 x 4096 x 1024 (1 round and 16)          46.7 -> 36.2
-//              4352 x 4096 x 256                            19.7 -> 16.3
 //              2048^3 (64 tiles)                            35.0 -> 18.8
+//   sixteenths, against eighths: 1024^3 (16 tiles) 6.9 -> 5.7, x 4096 19.8 -> 15.5,
+//              4352 x 4096 x 1024 33.6 -> 33.1
+//   eighths, against quarters: 5888 x 5888 x 1664 92.7 -> 90.6, 4352 x 4096 x 1024
+//              34.4 -> 32.8, 1024 x 2048 x 1024 (32 tiles) 9.3 -> 7.7, 256 x 256 x
+//              1024 8.1 -> 6.2
 //   halves     2560^3 (100 tiles)                           44.2 -> 34.6
 //              4864 x 4864 x 1024 (1 round and 105)         48.4 -> 45.0
-//   K no multiple of the quarters' 64: halves, 5888 x 5888 x 1632 107.6 -> 100.3
-// 256x128x64 s3 (halves are the same 128 x 128 parts): 2304 x 4096 x 2048 (1 round
-// and 32) 50.2 -> 42.8, 2048^3 (128 tiles) 23.2 -> 19.6.
+//   K no multiple of the smaller parts' 64: halves, 5888 x 5888 x 1632 107.6 -> 100.3
+// 256x128x64 s3 (its parts are the same blocks): halves at 2048^3 (128
+// tiles) 23.2 -> 19.6; quarters against halves at 2304 x 4096 x 2048 (1 round and 32)
+// 41.0 -> 38.1, whole 50.2.
 int tailParts(int rem, int slots, int K, int most) {
     if (rem == 0) return 1;
-    if (most >= 4 && K % 64 == 0 && 4 * rem <= slots) return 4;
+    if (K % 64 == 0)
+        for (int parts = most; parts >= 4; parts /= 2)
+            if (parts * rem <= slots) return parts;
     if (most >= 2 && 2 * rem <= slots) return 2;
     return 1;
 }

@@ -780,13 +780,17 @@ struct TailTiles {
     static constexpr int kLdsBytes = 0;
 };
 
-// 128 x 128 parts: BK = 64 and eight 32 x 64 wave tiles on the uniform loop, so that
-// the two wavefronts of a SIMD hide each other's barriers and LDS latency. At 2048^3
-// (one part per CU) 18.8 us, of which about 5 are launch, first fetch and epilogue;
-// 64 x 32 wave tiles 19.1, BK = 32 19.9, the ping-pong loop 20.6 (its memory phase
-// outlasts its 256-cycle matrix phase), deeper rings within 1%.
-struct TailQuarter {
-    using Blk = GemmBlock<128, 128, 64, 32, 64, 3, 1>;
+// The parts below a half: BK = 64 and eight wave tiles on the uniform loop, so that
+// the two wavefronts of a SIMD hide each other's barriers and LDS latency.
+//  * 128 x 128, wave tiles of 32 x 64: at 2048^3 (one part per CU) 18.8 us, of which
+//    about 5 are launch, first fetch and epilogue; 64 x 32 wave tiles 19.1, BK = 32
+//    19.9, the ping-pong loop 20.6 (its memory phase outlasts its 256-cycle matrix
+//    phase), deeper rings within 1%.
+//  * 64 x 128, wave tiles of 32 x 32; a fourth ring stage measured within 1%.
+//  * 64 x 64, wave tiles of 16 x 32; with six ring stages up to 9% slower.
+template <int BM, int BN, int WM, int WN, int STAGES>
+struct TailPart {
+    using Blk = GemmBlock<BM, BN, 64, WM, WN, STAGES, 1>;
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int N, int K) {
@@ -795,19 +799,26 @@ struct TailQuarter {
         blk.template store<NT>(C, N);
     }
 };
+using Part128x128 = TailPart<128, 128, 32, 64, 3>;
+using Part64x128 = TailPart<64, 128, 32, 32, 3>;
+using Part64x64 = TailPart<64, 64, 16, 32, 4>;
 
 template <>
 struct TailTiles<256, 256, 32> {
-    static constexpr int kParts = 4;
+    static constexpr int kParts = 16;
     using Half = GemmBlock<128, 256, 32, 64, 64, 3, 1>;
-    static constexpr int kLdsBytes = TailQuarter::Blk::T::kLdsBytes > Half::T::kLdsBytes
-                                         ? TailQuarter::Blk::T::kLdsBytes
-                                         : Half::T::kLdsBytes;
+    static constexpr int kLdsBytes = Part128x128::Blk::T::kLdsBytes;
+    static_assert(Half::T::kLdsBytes <= kLdsBytes && Part64x128::Blk::T::kLdsBytes <= kLdsBytes &&
+                  Part64x64::Blk::T::kLdsBytes <= kLdsBytes, "the quarters need the most LDS");
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int part, int parts, int N, int K) {
-        if (parts == 4) {
-            TailQuarter::run<NT>(lds, A, B, C, row + 128 * (part / 2), col + 128 * (part % 2), N, K);
+        if (parts == 16) {
+            Part64x64::run<NT>(lds, A, B, C, row + 64 * (part / 4), col + 64 * (part % 4), N, K);
+        } else if (parts == 8) {
+            Part64x128::run<NT>(lds, A, B, C, row + 64 * (part / 2), col + 128 * (part % 2), N, K);
+        } else if (parts == 4) {
+            Part128x128::run<NT>(lds, A, B, C, row + 128 * (part / 2), col + 128 * (part % 2), N, K);
         } else {
             Half blk(lds, A, B, row + 128 * part, col, N, K);
             pingPongLoop(blk, K / 32);
@@ -818,12 +829,18 @@ struct TailTiles<256, 256, 32> {
 
 template <>
 struct TailTiles<256, 128, 64> {
-    static constexpr int kParts = 2;
-    static constexpr int kLdsBytes = TailQuarter::Blk::T::kLdsBytes;
+    static constexpr int kParts = 8;
+    static constexpr int kLdsBytes = Part128x128::Blk::T::kLdsBytes;
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int part, int parts, int N, int K) {
-        TailQuarter::run<NT>(lds, A, B, C, row + 128 * part, col, N, K);
+        if (parts == 8) {
+            Part64x64::run<NT>(lds, A, B, C, row + 64 * (part / 2), col + 64 * (part % 2), N, K);
+        } else if (parts == 4) {
+            Part64x128::run<NT>(lds, A, B, C, row + 64 * part, col, N, K);
+        } else {
+            Part128x128::run<NT>(lds, A, B, C, row + 128 * part, col, N, K);
+        }
     }
 };
 
@@ -858,7 +875,7 @@ void gemmMfmaPingPongKernel(const _Float16* __restrict__ A, const _Float16* __re
         // The tail tiles are the last of the launch order; the parts of one tile
         // are neighbours and share an XCD.
         const int id = xcdRemap(blockIdx.x - wholeTiles, partTiles);
-        const int shift = parts / 2;  // parts is 2 or 4
+        const int shift = __builtin_ctz(parts);  // parts is a power of two
         tileOf<BM, BN, GROUPM>(wholeTiles + (id >> shift), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
         Tail::template run<NT>(lds, A, B, C, row, col, id & (parts - 1), parts, N, K);
     }

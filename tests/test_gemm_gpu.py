@@ -316,11 +316,11 @@ def test_c_at_the_non_temporal_threshold_bit_exact(M, N, K):
 
 
 # Output tiles of 256 x 256 around the tail rule's edges on 256 CUs: up to a
-# quarter round is cut into quarter tiles (K a multiple of 64), up to half a round
-# into half tiles; alone and behind a whole round. The last two grids start phased
+# sixteenth, an eighth or a quarter of a round is cut into as many parts (K a
+# multiple of 64), up to half a round into halves; alone and behind a whole round. The last two grids start phased
 # (three whole rounds).
 @pytest.mark.parametrize("tiles_m,tiles_n,K", [
-    (1, 1, 64), (1, 1, 96), (8, 8, 448), (8, 8, 96), (13, 5, 64), (13, 5, 480), (16, 8, 192), (43, 3, 64),
+    (1, 1, 64), (1, 1, 96), (1, 1, 576), (4, 4, 384), (17, 1, 64), (8, 4, 320), (11, 3, 64), (8, 8, 448), (8, 8, 96), (13, 5, 64), (13, 5, 480), (16, 8, 192), (43, 3, 64),
     (257, 1, 64), (257, 1, 32), (20, 16, 256), (107, 3, 128), (24, 16, 64), (77, 5, 64), (24, 32, 64), (32, 27, 64)])
 def test_ping_pong_tail_tiles_bit_exact(tiles_m, tiles_n, K):
     M, N = 256 * tiles_m, 256 * tiles_n
