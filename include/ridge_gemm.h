@@ -76,7 +76,10 @@ int ridge_gemm_divides(int i, int M, int N, int K);
 /* C = A * B with variant i. A: M x K, B: K x N, C: M x N, all row-major FP16 in
  * device memory, 16-byte aligned. Returns a hipError_t value: 0 on a successful
  * enqueue, 1 (hipErrorInvalidValue) on a bad index, shape or pointer, otherwise
- * the launch error. The reference's KernelVariant::launch (gemm-mma.cu:19-43). */
+ * the launch error. The reference's KernelVariant::launch (gemm-mma.cu:19-43).
+ * Where the row's tiles would leave most CUs idle (a small grid, or the last partial
+ * round of a ping-pong row) they run in smaller blocks of 512 threads within the same
+ * launch; the row's fields describe its own tile. */
 int ridge_gemm_launch(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
 
 /* Writes the variant table as CSV (header then one row per variant) into buf.

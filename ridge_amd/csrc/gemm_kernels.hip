@@ -64,22 +64,99 @@ struct SlotCache {
     }
 };
 
+// CUs of the current device, cached per device; 0 when it cannot be asked.
+int deviceCus() {
+    static std::atomic<int> cache[kMaxDevices];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+    const int cached = cache[dev].load(std::memory_order_relaxed);
+    if (cached > 0) return cached;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    cache[dev].store(cus, std::memory_order_relaxed);
+    return cus;
+}
+
+// The block (ridge::SmallGridPart) in which a uniform or persistent row runs a grid of
+// at most half as many of its tiles as the device has CUs, 0 for the row's own tile:
+// the smallest whose workgroups still fit one round. Own tile -> parts, operands cold:
+// 128x128x64 s4 persistent 1024^3 9.1 -> 5.6 us, 2048 x 1024 x 1024 9.1 -> 7.5, 1024 x
+// 1024 x 4096 25.4 -> 15.9; 128x128x64 s2 1024^3 11.7 -> 5.6; 128x64x64 s3 512^3 4.9 ->
+// 3.8; 64x128x128 s3 persistent 8192 x 128 x 4096 (128 tiles) 19.7 -> 15.3; 256x256x64
+// s2 1024 x 2048 x 1024 24.9 -> 7.7.
+template <int BM, int BN>
+int smallGridPart(int M, int N, int K) {
+    if (BM * BN <= 64 * 64 || K % 64 != 0) return 0;
+    const int cus = deviceCus();
+    if ((M / BM) * (N / BN) > cus / 2) return 0;
+    if ((M / 64) * (N / 64) <= cus) return 1;
+    if (BN >= 128 && (M / 64) * (N / 128) <= cus) return 2;
+    if (BM >= 128 && BN >= 128 && (M / 128) * (N / 128) <= cus) return 3;
+    return 0;
+}
+
+template <int PART>
+struct PartGrid {
+    ridge::TileOrder order;
+    dim3 grid;
+    PartGrid(int M, int N) {
+        using P = typename ridge::SmallGridPart<PART>::Part;
+        order = ridge::tileOrder<P::kBM, P::kBN, ridge::kPartGroupM>(M, N);
+        grid = dim3((unsigned)((M / P::kBM) * (N / P::kBN)));
+    }
+};
+
+template <int BM, int BN, int BK, int WM, int WN, int S, int G, int PART>
+void enqueuePersistentParts(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
+                            hipStream_t stream) {
+    const PartGrid<PART> g(M, N);
+    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, PART>), g.grid,
+                       dim3(ridge::kPartThreads), 0, stream, A, B, C, M, N, K, g.order.group, g.order.lastRows, 0u, 0,
+                       0, 0);
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int S, int G, int PART>
+void enqueueUniformParts(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
+    const PartGrid<PART> g(M, N);
+    hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, false, PART>), g.grid,
+                       dim3(ridge::kPartThreads), 0, stream, A, B, C, M, N, K, g.order.group, g.order.lastRows, 0u);
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
 hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
     using P = ridge::PersistentTraits<BM, BN, BK, WM, WN, S, G>;
+    const auto* a = static_cast<const _Float16*>(A);
+    const auto* b = static_cast<const _Float16*>(B);
+    auto* c = static_cast<_Float16*>(C);
+    const int part = smallGridPart<BM, BN>(M, N, K);
+    if (part == 1) {
+        enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 1>(a, b, c, M, N, K, stream);
+        return hipGetLastError();
+    }
+    if constexpr (BN >= 128) {
+        if (part == 2) {
+            enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 2>(a, b, c, M, N, K, stream);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (BM >= 128 && BN >= 128) {
+        if (part == 3) {
+            enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 3>(a, b, c, M, N, K, stream);
+            return hipGetLastError();
+        }
+    }
     static SlotCache cache;
     hipError_t err;
     const int resident = cache.of(
-        reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), P::kThreads, &err);
+        reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, 0>), P::kThreads,
+        &err);
     if (resident <= 0) return err;
     // Every workgroup must own at least one tile (the kernel's tile count per
     // workgroup assumes it).
     const int tiles = (M / BM) * (N / BN);
     const int grid = tiles < resident ? tiles : resident;
     const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
-    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), dim3((unsigned)grid),
-                       dim3(P::kThreads), 0, stream, static_cast<const _Float16*>(A),
-                       static_cast<const _Float16*>(B), static_cast<_Float16*>(C), M, N, K, order.group,
+    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, 0>), dim3((unsigned)grid),
+                       dim3(P::kThreads), 0, stream, a, b, c, M, N, K, order.group,
                        order.lastRows, ridge::reciprocalOf(K / BK), grid, tiles / grid, tiles % grid);
     return hipGetLastError();
 }
@@ -146,7 +223,26 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
                            order.lastRows, whole, partTiles,
                            parts | phaseWidth(whole, slots, K) << 8);
     } else {
-        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
+        if constexpr (!NT && BM * BN > 64 * 64) {
+            const int part = smallGridPart<BM, BN>(M, N, K);
+            if (part == 1) {
+                enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 1>(A, B, C, M, N, K, stream);
+                return hipGetLastError();
+            }
+            if constexpr (BN >= 128) {
+                if (part == 2) {
+                    enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 2>(A, B, C, M, N, K, stream);
+                    return hipGetLastError();
+                }
+            }
+            if constexpr (BM >= 128 && BN >= 128) {
+                if (part == 3) {
+                    enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 3>(A, B, C, M, N, K, stream);
+                    return hipGetLastError();
+                }
+            }
+        }
+        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT, 0>), dim3((unsigned)tiles), block, 0,
                            stream, A, B, C, M, N, K, order.group, order.lastRows, ridge::reciprocalOf(K / BK));
     }
     return hipGetLastError();

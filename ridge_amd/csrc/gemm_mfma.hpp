@@ -628,38 +628,99 @@ __device__ __forceinline__ void uniformLoop(Blk& blk, int numK) {
     barrierLds();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
+// Blocks that stand in for a row's tiles where those leave CUs idle: the parts of a
+// ping-pong row's last round (below) and grids of few tiles. BK = 64 and eight wave
+// tiles on the uniform loop, so that the two wavefronts of a SIMD hide each other's
+// barriers and LDS latency.
+//  * 128 x 128, wave tiles of 32 x 64: at 2048^3 (one part per CU) 18.8 us, of which
+//    about 5 are launch, first fetch and epilogue; 64 x 32 wave tiles 19.1, BK = 32
+//    19.9, the ping-pong loop 20.6 (its memory phase outlasts its 256-cycle matrix
+//    phase), deeper rings within 1%.
+//  * 64 x 128, wave tiles of 32 x 32; a fourth ring stage measured within 1%.
+//  * 64 x 64, wave tiles of 16 x 32; with six ring stages up to 9% slower.
+template <int BM, int BN, int WM, int WN, int STAGES>
+struct TilePart {
+    static constexpr int kBM = BM, kBN = BN;
+    using Blk = GemmBlock<BM, BN, 64, WM, WN, STAGES, 1>;
+    template <bool NT>
+    static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
+                                               int row, int col, int N, int K) {
+        Blk blk(lds, A, B, row, col, N, K);
+        uniformLoop<false, true>(blk, K / 64);
+        blk.template store<NT>(C, N);
+    }
+};
+using Part128x128 = TilePart<128, 128, 32, 64, 3>;
+using Part64x128 = TilePart<64, 128, 32, 32, 3>;
+using Part64x64 = TilePart<64, 64, 16, 32, 4>;
+
+// Kernels that carry a row's template arguments run a whole small grid in blocks of
+// PART (smallGridPart in gemm_kernels.hip): 0 is the row's own tile.
+template <int PART>
+struct SmallGridPart;
+template <>
+struct SmallGridPart<1> {
+    using Part = Part64x64;
+};
+template <>
+struct SmallGridPart<2> {
+    using Part = Part64x128;
+};
+template <>
+struct SmallGridPart<3> {
+    using Part = Part128x128;
+};
+constexpr int kPartThreads = 512;
+constexpr int kPartGroupM = 8;
+
+template <int PART>
+__device__ __forceinline__ void runSmallGrid(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
+                                             TileOrder order) {
+    using P = typename SmallGridPart<PART>::Part;
+    static_assert(P::Blk::T::kThreads == kPartThreads, "parts have eight wavefronts");
+    __shared__ __attribute__((aligned(1024))) char lds[P::Blk::T::kLdsBytes];
+    int row, col;
+    const int tiles = (M / P::kBM) * (N / P::kBN);
+    tileOf<P::kBM, P::kBN, kPartGroupM>(xcdRemap(blockIdx.x, tiles), M, N, order, row, col);
+    P::template run<false>(lds, A, B, C, row, col, N, K);
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT, int PART>
+__global__ __launch_bounds__(PART != 0 ? kPartThreads : (BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                     _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
                     uint32_t lastRowsReciprocal, uint32_t numKReciprocal) {
-    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
-    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
-    int row, col;
-    const int tiles = (M / BM) * (N / BN);  // = gridDim.x, which would be a load
-    tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
-    GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
-    const int numK = K / BK;
-    // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
-    // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
-    // Cold, when the first touch of every K slice comes from HBM, workgroups in
-    // lockstep all request the same K slice of their panels at once (A's slice
-    // strided by a row); staggered, they request different slices. Measured at
-    // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
-    // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
-    // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
-    // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
-    // long K loops, which gained nothing. Only the summation order of the K tiles
-    // changes.
-    constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
-    if constexpr (kStagger) {
-        if (numK <= 32) blk.kStart = (int)divide((uint32_t)(row / BM + col / BN), numK, numKReciprocal).rem;
-    }
+    if constexpr (PART != 0) {
+        runSmallGrid<PART>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal});
+    } else {
+        using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+        __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
+        int row, col;
+        const int tiles = (M / BM) * (N / BN);  // = gridDim.x, which would be a load
+        tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
+        GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
+        const int numK = K / BK;
+        // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
+        // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
+        // Cold, when the first touch of every K slice comes from HBM, workgroups in
+        // lockstep all request the same K slice of their panels at once (A's slice
+        // strided by a row); staggered, they request different slices. Measured at
+        // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
+        // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
+        // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
+        // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
+        // long K loops, which gained nothing. Only the summation order of the K tiles
+        // changes.
+        constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
+        if constexpr (kStagger) {
+            if (numK <= 32) blk.kStart = (int)divide((uint32_t)(row / BM + col / BN), numK, numKReciprocal).rem;
+        }
 
-    // The 8-wave rows (two stages, 256 registers per lane) keep the general form
-    // of the loop only: the second copy made them spill.
-    uniformLoop<kStagger, (T::kWaves <= 4)>(blk, numK);
-    blk.template store<NT>(C, N);
+        // The 8-wave rows (two stages, 256 registers per lane) keep the general form
+        // of the loop only: the second copy made them spill.
+        uniformLoop<kStagger, (T::kWaves <= 4)>(blk, numK);
+        blk.template store<NT>(C, N);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -779,29 +840,6 @@ struct TailTiles {
     static constexpr int kParts = 1;      // the most parts of one tile
     static constexpr int kLdsBytes = 0;
 };
-
-// The parts below a half: BK = 64 and eight wave tiles on the uniform loop, so that
-// the two wavefronts of a SIMD hide each other's barriers and LDS latency.
-//  * 128 x 128, wave tiles of 32 x 64: at 2048^3 (one part per CU) 18.8 us, of which
-//    about 5 are launch, first fetch and epilogue; 64 x 32 wave tiles 19.1, BK = 32
-//    19.9, the ping-pong loop 20.6 (its memory phase outlasts its 256-cycle matrix
-//    phase), deeper rings within 1%.
-//  * 64 x 128, wave tiles of 32 x 32; a fourth ring stage measured within 1%.
-//  * 64 x 64, wave tiles of 16 x 32; with six ring stages up to 9% slower.
-template <int BM, int BN, int WM, int WN, int STAGES>
-struct TailPart {
-    using Blk = GemmBlock<BM, BN, 64, WM, WN, STAGES, 1>;
-    template <bool NT>
-    static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
-                                               int row, int col, int N, int K) {
-        Blk blk(lds, A, B, row, col, N, K);
-        uniformLoop<false, true>(blk, K / 64);
-        blk.template store<NT>(C, N);
-    }
-};
-using Part128x128 = TailPart<128, 128, 32, 64, 3>;
-using Part64x128 = TailPart<64, 128, 32, 32, 3>;
-using Part64x64 = TailPart<64, 64, 16, 32, 4>;
 
 template <>
 struct TailTiles<256, 256, 32> {
@@ -935,11 +973,9 @@ struct PersistentTraits {
 };
 
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
-__global__ __launch_bounds__(((BM / WM) * (BN / WN) + kPersistentLoaders) * kWaveSize)
-void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
-                              _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
-                              uint32_t lastRowsReciprocal, uint32_t numKReciprocal, int grid, int tilesEach,
-                              int tilesMore) {
+__device__ __forceinline__ void persistentWalk(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
+                                               TileOrder order, uint32_t numKReciprocal, int grid, int tilesEach,
+                                               int tilesMore) {
     using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using P = PersistentTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
     using Blk = GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM>;
@@ -952,7 +988,6 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int lane = threadIdx.x % kWaveSize;
     const int self = xcdRemap(blockIdx.x, grid);
-    const TileOrder order = {groupReciprocal, lastRowsReciprocal};
     const int numK = K / BK;
     // The launcher makes grid <= the tile count, so every workgroup has a tile:
     // tilesEach, and one more for the first tilesMore workgroups.
@@ -1115,6 +1150,20 @@ void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __
         for (; g0 + U < G; g0 += U) pass(g0, std::true_type{});
     }
     for (; g0 < G; g0 += U) pass(g0, std::false_type{});
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, int PART>
+__global__ __launch_bounds__(PART != 0 ? kPartThreads : ((BM / WM) * (BN / WN) + kPersistentLoaders) * kWaveSize)
+void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
+                              _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
+                              uint32_t lastRowsReciprocal, uint32_t numKReciprocal, int grid, int tilesEach,
+                              int tilesMore) {
+    if constexpr (PART != 0) {
+        runSmallGrid<PART>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal});
+    } else {
+        persistentWalk<BM, BN, BK, WM, WN, STAGES, GROUPM>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal},
+                                                           numKReciprocal, grid, tilesEach, tilesMore);
+    }
 }
 
 }  // namespace ridge

@@ -347,6 +347,21 @@ def test_launch_order_with_ragged_groups_bit_exact(tiles_m, tiles_n):
         assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
 
 
+# Grids around the small-grid rule's edges on 256 CUs for every tile size: as 64 x 64
+# blocks (256 of them at 1024 x 1024), 64 x 128, 128 x 128, and one tile too many.
+@pytest.mark.parametrize("M,N,K", [(256, 256, 64), (1024, 1024, 192), (1024, 1280, 64), (2048, 1024, 64),
+                                   (2048, 1280, 64), (2048, 2048, 128), (4096, 2048, 64), (4096, 2304, 64),
+                                   (8192, 256, 320), (256, 8448, 64), (1024, 1024, 96)])
+def test_small_grids_bit_exact_every_variant(M, N, K):
+    Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + 11 * N + K)
+    A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
+    for v in G.variants():
+        if not v.divides(M, N, K):
+            continue
+        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
+        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+
+
 def _persistent_edge_shapes(v):
     """Shapes that drive the persistent schedule's control flow to its edges."""
     BM, BN, BK, S = v.BM, v.BN, v.BK, v.stages
