@@ -85,7 +85,7 @@ int deviceCus() {
 // s2 1024 x 2048 x 1024 24.9 -> 7.7.
 template <int BM, int BN>
 int smallGridPart(int M, int N, int K) {
-    if (BM * BN <= 64 * 64 || K % 64 != 0) return 0;
+    if (BM * BN <= 64 * 64 || !ridge::partsFit(N, K)) return 0;
     const int cus = deviceCus();
     if ((M / BM) * (N / BN) > cus / 2) return 0;
     if ((M / 64) * (N / 64) <= cus) return 1;
@@ -176,12 +176,14 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
 //   halves     2560^3 (100 tiles)                           44.2 -> 34.6
 //              4864 x 4864 x 1024 (1 round and 105)         48.4 -> 45.0
 //   K no multiple of the smaller parts' 64: halves, 5888 x 5888 x 1632 107.6 -> 100.3
+// The halves of the 256x256x32 rows keep the row's BK and with it the row's offset
+// bound; those of 256x128x64 are of the smaller parts' BK, which is also the row's.
 // 256x128x64 s3 (its parts are the same blocks): halves at 2048^3 (128
 // tiles) 23.2 -> 19.6; quarters against halves at 2304 x 4096 x 2048 (1 round and 32)
 // 41.0 -> 38.1, whole 50.2.
-int tailParts(int rem, int slots, int K, int most) {
+int tailParts(int rem, int slots, int N, int K, int most) {
     if (rem == 0) return 1;
-    if (K % 64 == 0)
+    if (ridge::partsFit(N, K))
         for (int parts = most; parts >= 4; parts /= 2)
             if (parts * rem <= slots) return parts;
     if (most >= 2 && 2 * rem <= slots) return 2;
@@ -215,7 +217,7 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
             &err);
         // A device that does not say its slots runs every tile whole.
         const int rem = slots > 0 ? tiles % slots : 0;
-        const int parts = tailParts(rem, slots, K, ridge::TailTiles<BM, BN, BK>::kParts);
+        const int parts = tailParts(rem, slots, N, K, ridge::TailTiles<BM, BN, BK>::kParts);
         const int whole = parts > 1 ? tiles - rem : tiles;
         const int partTiles = (tiles - whole) * parts;
         hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>),
@@ -341,8 +343,7 @@ int ridge_gemm_divides(int i, int M, int N, int K) {
     if (M % e.BM || N % e.BN || K % e.BK) return 0;
     // The grid is one-dimensional and offsets inside the kernel are 32-bit.
     if ((long long)(M / e.BM) * (N / e.BN) > 0x7fffffffLL) return 0;
-    if ((long long)e.BM * K > 0x7fffffffLL || (long long)e.BK * N > 0x7fffffffLL) return 0;
-    return 1;
+    return ridge::tileOffsetsFit(e.BM, e.BK, N, K) ? 1 : 0;
 }
 
 int ridge_gemm_launch(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream) {

@@ -43,7 +43,8 @@
 //
 // Preconditions (checked by the host launcher, never by the kernel): M % BM ==
 // N % BN == K % BK == 0 and K >= BK; BM * K, BK * N and the tile count below 2^31
-// (tile offsets are 32-bit); 16-byte aligned A, B, C.
+// (tile offsets are 32-bit), BM and BK being those of every block that the launch
+// runs, the row's tile or its parts (TilePart); 16-byte aligned A, B, C.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -196,8 +197,12 @@ __device__ __forceinline__ void globalLoadLds16(const void* base, uint32_t offse
 
 // LDS byte address of a __shared__ object, as a wave-uniform scalar.
 // Byte offset of 16-byte chunk `chunk` of row `row` in an FP16 tile whose rows are
-// `ld` elements apart. Unsigned 32-bit arithmetic: the launcher admits only shapes
-// with BM * K and BK * N below 2^31, so every tile offset is below 2^32.
+// `ld` elements apart. Unsigned 32-bit arithmetic: the launcher runs a BM x BN x BK
+// block only on shapes that it fits (tileOffsetsFit), so every tile offset is below 2^32.
+constexpr bool tileOffsetsFit(int BM, int BK, int N, int K) {
+    return (long long)BM * K <= 0x7fffffffLL && (long long)BK * N <= 0x7fffffffLL;
+}
+
 __device__ __forceinline__ uint32_t tileOffset(int row, int ld, int chunk) {
     return ((uint32_t)row * (uint32_t)ld + (uint32_t)chunk * 8u) * 2u;
 }
@@ -638,15 +643,24 @@ __device__ __forceinline__ void uniformLoop(Blk& blk, int numK) {
 //    phase), deeper rings within 1%.
 //  * 64 x 128, wave tiles of 32 x 32; a fourth ring stage measured within 1%.
 //  * 64 x 64, wave tiles of 16 x 32; with six ring stages up to 9% slower.
+// A part's tile offsets have a bound of their own (partsFit): a row with BK = 32 is
+// admitted up to twice the N that a part's 64 rows of B allow.
+constexpr int kPartBK = 64;
+constexpr int kPartMostBM = 128;
+constexpr bool partsFit(int N, int K) {
+    return K % kPartBK == 0 && tileOffsetsFit(kPartMostBM, kPartBK, N, K);
+}
+
 template <int BM, int BN, int WM, int WN, int STAGES>
 struct TilePart {
+    static_assert(BM <= kPartMostBM, "partsFit bounds the offsets of blocks of at most this many rows");
     static constexpr int kBM = BM, kBN = BN;
-    using Blk = GemmBlock<BM, BN, 64, WM, WN, STAGES, 1>;
+    using Blk = GemmBlock<BM, BN, kPartBK, WM, WN, STAGES, 1>;
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int N, int K) {
         Blk blk(lds, A, B, row, col, N, K);
-        uniformLoop<false, true>(blk, K / 64);
+        uniformLoop<false, true>(blk, K / kPartBK);
         blk.template store<NT>(C, N);
     }
 };

@@ -469,6 +469,33 @@ def test_largest_n_the_offset_guard_admits_is_exact_on_bk128_persistent_rows():
         torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("N", [33497344, 34087168])
+def test_wide_rows_beside_the_offset_bound_of_their_parts_are_exact(N):
+    """One row of 256 x 256 tiles, 33 more than whole rounds of 256 CUs, at an N where
+    the last round runs as quarters (BK = 64) and at one where their B offsets would
+    pass 32 bits. A[i, k] = 1 where k = i (mod 64) and B[k, j] = 1 where k + j = 0
+    (mod 3), so C[i, j] is B[i mod 64, j]; an offset of B's last rows less 2^32 bytes
+    reads another class. Checked on the device, every output; C is about 17 GB."""
+    M, K = 256, 64
+    rows = [v for v in G.variants() if v.schedule == 1 and (v.BM, v.BN, v.BK) == (256, 256, 32)]
+    assert len(rows) == 8 and all(v.divides(M, N, K) for v in rows)
+    A = (torch.arange(K, device=DEV)[None, :] == torch.arange(M, device=DEV)[:, None] % K).to(torch.float16)
+    jm3 = torch.arange(N, device=DEV, dtype=torch.int32) % 3
+    B = torch.empty((K, N), dtype=torch.float16, device=DEV)
+    for k in range(K):
+        B[k] = (jm3 == (-k) % 3).to(torch.float16)
+    C = torch.empty((M, N), dtype=torch.float16, device=DEV)
+    for v in rows:
+        print("  %s at %dx%dx%d" % (v.label(), M, N, K), flush=True)
+        C.fill_(float("nan"))
+        assert G.launch(v.index, A, B, C, M, N, K) == 0
+        torch.cuda.synchronize()
+        bad = sum(int((C[i] != B[i % K]).sum().item()) for i in range(M))
+        assert bad == 0, "%s at N = %d: %d of %d outputs differ" % (v.label(), N, bad, M * N)
+    del A, B, C, jm3
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 1024), (4096, 4096, 4096), (8192, 8192, 128),
                                    (16384, 128, 8192)])
 def test_baseline_configs_uniform_inputs(M, N, K):

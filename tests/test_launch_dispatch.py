@@ -1,0 +1,136 @@
+"""Which kernel, grid and arguments a launch takes, on the CPU: the kernel library
+runs in a child process on a stand-in for the HIP runtime, which records the launches
+instead of making them and can be told to refuse a device query."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from ridge_amd import gemm as G
+
+FAKE_HIP = r"""
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+typedef struct { uint32_t x, y, z; } dim3_t;
+static struct { const void* fn; const char* name; } kernels[4096];
+static int count, error;
+static dim3_t grid, block;
+static size_t shared;
+static void* stream;
+
+void** __hipRegisterFatBinary(const void* data) { static void* handle; (void)data; return &handle; }
+void __hipUnregisterFatBinary(void** modules) { (void)modules; }
+void __hipRegisterFunction(void** modules, const void* host, char* device, const char* name, unsigned limit,
+                           void* tid, void* bid, dim3_t* b, dim3_t* g, int* w) {
+    (void)modules; (void)device; (void)limit; (void)tid; (void)bid; (void)b; (void)g; (void)w;
+    if (count < 4096) { kernels[count].fn = host; kernels[count++].name = name; }
+}
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t n, void* s) {
+    grid = g; block = b; shared = n; stream = s;
+    return 0;
+}
+int __hipPopCallConfiguration(dim3_t* g, dim3_t* b, size_t* n, void** s) {
+    *g = grid; *b = block; *n = shared; *s = stream;
+    return 0;
+}
+int hipLaunchKernel(const void* fn, dim3_t g, dim3_t b, void** args, size_t n, void* s) {
+    const char* name = "";
+    (void)n; (void)s;
+    for (int i = 0; i < count; ++i)
+        if (kernels[i].fn == fn) name = kernels[i].name;
+    const int ints = strstr(name, "PingPong") ? 8 : strstr(name, "Persistent") ? 9 : 6;
+    printf("{\"kernel\": \"%s\", \"grid\": %u, \"block\": %u, \"args\": [", name, g.x, b.x);
+    for (int i = 0; i < ints; ++i) printf("%s%u", i ? ", " : "", *(uint32_t*)args[3 + i]);
+    printf("]}\n");
+    fflush(stdout);
+    return 0;
+}
+static int refused(const char* what) {
+    const char* names = getenv("FAKE_HIP_REFUSES");
+    if (names == 0 || strstr(names, what) == 0) return 0;
+    error = 101;
+    return 1;
+}
+int hipGetDevice(int* device) { if (refused("hipGetDevice")) return 101; *device = 0; return 0; }
+int hipDeviceGetAttribute(int* value, int attribute, int device) {
+    (void)attribute; (void)device;
+    if (refused("hipDeviceGetAttribute")) return 101;
+    *value = 256;
+    return 0;
+}
+int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* blocks, const void* fn, int threads, size_t n) {
+    (void)fn; (void)threads; (void)n;
+    if (refused("hipOccupancy")) return 101;
+    *blocks = 1;
+    return 0;
+}
+int hipGetLastError(void) { const int e = error; error = 0; return e; }
+"""
+
+# Loads the stand-in first and globally, so that the library's references bind to it.
+CHILD = r"""
+import ctypes, json, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+L = ctypes.CDLL(sys.argv[2])
+L.ridge_gemm_launch.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+for call in json.load(sys.stdin):
+    rc = L.ridge_gemm_launch(call[0], 4096, 4096, 4096, call[1], call[2], call[3], None)
+    print(json.dumps({"rc": rc}), flush=True)
+"""
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    d = tmp_path_factory.mktemp("fake_hip")
+    src, so = d / "fake_hip.c", d / "libfake_hip.so"
+    src.write_text(FAKE_HIP)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    return str(so)
+
+
+def launches(fake_hip, calls, refuses=""):
+    """[(return code, the launches made)] of calls (variant index, M, N, K)."""
+    env = dict(os.environ, FAKE_HIP_REFUSES=refuses)
+    p = subprocess.run([sys.executable, "-c", CHILD, fake_hip, G.LIB_PATH], input=json.dumps(calls), env=env,
+                       capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
+    out, made = [], []
+    for line in p.stdout.splitlines():
+        r = json.loads(line)
+        if "rc" in r:
+            out.append((r["rc"], made))
+            made = []
+        else:
+            made.append(r)
+    assert len(out) == len(calls)
+    return out
+
+
+def rows(schedule=None, **fields):
+    return [v for v in G.variants() if (schedule is None or v.schedule == schedule) and
+            all(getattr(v, k) == x for k, x in fields.items())]
+
+
+def ping_pong_parts(launch):
+    """(whole tiles, workgroups of parts, parts per tile) of a ping-pong launch."""
+    whole, part_tiles, parts_and_phase = launch["args"][5:8]
+    return whole, part_tiles, parts_and_phase & 0xff
+
+
+# 130849 and 133153 tiles: 33 behind whole rounds of 256, which fit one round as
+# quarters. The quarters have BK = 64, and their last B row starts 63 * N * 2 bytes
+# into the tile: 32 bits hold that for the first N and not for the second.
+@pytest.mark.parametrize("N,parts", [(33497344, 4), (34087168, 2)])
+def test_parts_whose_b_offsets_pass_32_bits_are_not_taken(fake_hip, N, parts):
+    wide = rows(1, BM=256, BN=256, BK=32)
+    assert len(wide) == 8
+    tiles = N // 256
+    for v, (rc, made) in zip(wide, launches(fake_hip, [(v.index, 256, N, 64) for v in wide])):
+        assert rc == 0 and len(made) == 1
+        assert ping_pong_parts(made[0]) == (tiles - 33, 33 * parts, parts), v.label()
+        # What the blocks address: BK rows of B (halves keep the row's 32).
+        assert (64 if parts >= 4 else 32) * N < 2 ** 31
