@@ -255,7 +255,8 @@ hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, in
     const auto* a = static_cast<const _Float16*>(A);
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
-    if ((size_t)M * N * 2 > ridge::kNonTemporalBytes)
+    constexpr bool pingPong = usesPingPong(ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kWaves, S);
+    if ((size_t)M * N * 2 > ridge::kNonTemporalBytes && !(pingPong && K < ridge::kNonTemporalPingPongK))
         return enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
     return enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);
 }

@@ -367,7 +367,16 @@ __device__ __forceinline__ void storeStaged(const float4_t (&acc)[TM][TN], RIDGE
 // non-temporal stores made the GEMM itself 10% faster, but it and a GEMM that
 // follows on C 14% slower together; at 5120 x 5120 (52 MB) 0 and 1% slower, at
 // 6144 x 6144 (75 MB) 1% and 2% faster.
+// A ping-pong row's C of a single 32-deep step stays cached too: there is no panel to
+// keep, and where launches write the same C again the MALL takes it. 256x256x32 rows at
+// K = 32, the mean of eight, one C | eight in turn, cached against non-temporal:
+// 8192 x 6144 19.1 against 23.3 | 22.4 against 23.1 us, 8192 x 8192 24.7 against 30.4 |
+// 30.3 against 30.5, 16384 x 8192 49.5 against 52.2 | 53.5 against 52.5, 8192 x 4352
+// 17.3 against 17.2 | 18.5 against 17.2. Non-temporal, rows lost up to 12% to the cached
+// stores of a kernel without the phased start; cached, none does. At K = 64 eight Cs in
+// turn are 3-12% faster non-temporal and one C between 10% faster and 9% slower.
 constexpr size_t kNonTemporalBytes = (size_t)64 << 20;
+constexpr int kNonTemporalPingPongK = 64;
 
 // Per-workgroup state and the operations both schedules are built from: the
 // output tile, the direct-to-LDS refill of a stage, the fragment reads of a

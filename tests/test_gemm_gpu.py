@@ -302,10 +302,11 @@ def test_random_divisible_shapes_uniform_inputs_every_variant(M, N, K):
         M, N, K, len(rows), worst_row[0], worst_row[2], worst_row[1]), flush=True)
 
 
-@pytest.mark.parametrize("M,N,K", [(8192, 4096, 64), (8192, 4352, 64)])
+@pytest.mark.parametrize("M,N,K", [(8192, 4096, 64), (8192, 4352, 64), (8192, 4352, 32)])
 def test_c_at_the_non_temporal_threshold_bit_exact(M, N, K):
     """A C of exactly 64 MiB (cached stores) and the next one above (non-temporal
-    stores): two instantiations of every uniform and ping-pong row."""
+    stores, but for ping-pong rows at K = 32): two instantiations of every uniform and
+    ping-pong row."""
     Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + N + K)
     A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
     for v in G.variants():

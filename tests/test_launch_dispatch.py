@@ -134,3 +134,15 @@ def test_parts_whose_b_offsets_pass_32_bits_are_not_taken(fake_hip, N, parts):
         assert ping_pong_parts(made[0]) == (tiles - 33, 33 * parts, parts), v.label()
         # What the blocks address: BK rows of B (halves keep the row's 32).
         assert (64 if parts >= 4 else 32) * N < 2 ** 31
+
+
+def test_c_above_64_mib_is_stored_non_temporally_but_for_a_single_32_deep_step(fake_hip):
+    """The kernels' bool template argument (Lb1E): true above 64 MiB of C, where
+    non-temporal stores are the faster ones; a ping-pong row's K of 32 is not."""
+    for v in rows(0) + rows(1):
+        shapes = [(8192, 4096, K) for K in (32, 64)] + [(8192, 6144, K) for K in (32, 64, 128)]
+        shapes = [s for s in shapes if v.divides(*s)]
+        for (M, N, K), (rc, made) in zip(shapes, launches(fake_hip, [(v.index,) + s for s in shapes])):
+            assert rc == 0 and len(made) == 1
+            nt = M * N * 2 > 64 << 20 and not (v.schedule == 1 and K < 64)
+            assert ("ELb1E" in made[0]["kernel"]) == nt, (v.label(), M, N, K, made[0]["kernel"])
