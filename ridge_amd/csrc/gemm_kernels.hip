@@ -64,14 +64,23 @@ struct SlotCache {
     }
 };
 
-// CUs of the current device, cached per device; 0 when it cannot be asked.
+// CUs of the current device, cached per device; 0 when it cannot be asked. Its callers
+// then run the row's own tiles, so the query's error is dropped: the launch reports its
+// own by hipGetLastError.
 int deviceCus() {
     static std::atomic<int> cache[kMaxDevices];
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+    if (hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    if (dev < 0 || dev >= kMaxDevices) return 0;
     const int cached = cache[dev].load(std::memory_order_relaxed);
     if (cached > 0) return cached;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
     cache[dev].store(cus, std::memory_order_relaxed);
     return cus;
 }
@@ -210,12 +219,9 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
     const dim3 block(T::kThreads);
     const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
     if constexpr (usesPingPong(T::kWaves, S)) {
-        static SlotCache cache;
-        hipError_t err;
-        const int slots = cache.of(
-            reinterpret_cast<const void*>(&ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>), T::kThreads,
-            &err);
-        // A device that does not say its slots runs every tile whole.
+        static_assert(2 * T::kLdsBytes > 163840, "a ping-pong row has one workgroup per CU");
+        const int slots = deviceCus();
+        // A device that does not say its CUs runs every tile whole.
         const int rem = slots > 0 ? tiles % slots : 0;
         const int parts = tailParts(rem, slots, N, K, ridge::TailTiles<BM, BN, BK>::kParts);
         const int whole = parts > 1 ? tiles - rem : tiles;

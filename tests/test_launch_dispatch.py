@@ -146,3 +146,17 @@ def test_c_above_64_mib_is_stored_non_temporally_but_for_a_single_32_deep_step(f
             assert rc == 0 and len(made) == 1
             nt = M * N * 2 > 64 << 20 and not (v.schedule == 1 and K < 64)
             assert ("ELb1E" in made[0]["kernel"]) == nt, (v.label(), M, N, K, made[0]["kernel"])
+
+
+@pytest.mark.parametrize("query", ["hipGetDevice", "hipDeviceGetAttribute", "hipOccupancy"])
+def test_a_launch_whose_device_query_fails_runs_its_own_tiles_and_succeeds(fake_hip, query):
+    """Uniform and ping-pong rows only choose smaller blocks by the device's CUs: where
+    those are not to be had, the launch is the whole grid of the row's tile, and the
+    query's error is not reported as the launch's."""
+    picked = rows(0) + rows(1)
+    M, N, K = 1024, 1024, 128
+    for v, (rc, made) in zip(picked, launches(fake_hip, [(v.index, M, N, K) for v in picked], query)):
+        assert rc == 0 and len(made) == 1, v.label()
+        if query != "hipOccupancy":
+            assert made[0]["grid"] == (M // v.BM) * (N // v.BN), v.label()
+            assert made[0]["block"] == v.threads, v.label()
