@@ -89,13 +89,14 @@ def read_variant_list():
 
 def parse_resource_remarks(text):
     """Maps (BM,BN,BK,WM,WN,S,G,persistent) -> resource dict from -Rpass-analysis
-    output; a row's kernel with non-temporal stores has "nt" behind its key, its
-    small-grid forms ("part", n)."""
+    output; a row's kernel with non-temporal stores has "nt" behind its key, and the
+    small-grid kernel of block n is ("part", n)."""
     out = {}
     cur = None
     name_re = re.compile(r"Function Name: (\S+)")
     tmpl_re = re.compile(
-        r"gemmMfma(PingPong|Persistent)?KernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E(?:Lb([01])E)?(?:Li(\d+)E)?")
+        r"gemmMfma(PingPong|Persistent)?KernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E(?:Lb([01])E)?")
+    part_re = re.compile(r"gemmMfmaSmallGridKernelILi(\d+)E")
     field_re = re.compile(r"remark:\s+([A-Za-z][A-Za-z /\[\]]*?):\s*(\S+)")
     for line in text.splitlines():
         m = name_re.search(line)
@@ -105,8 +106,9 @@ def parse_resource_remarks(text):
                    if t else None)
             if cur is not None and t.group(9) == "1":
                 cur += ("nt",)  # the non-temporal form of a row: gated, not in the table
-            if cur is not None and t.group(10) not in (None, "0"):
-                cur += ("part", int(t.group(10)))  # a row's small-grid form: likewise
+            part = part_re.search(m.group(1))
+            if part:
+                cur = ("part", int(part.group(1)))  # likewise
             if cur is not None:
                 out[cur] = {}
             continue

@@ -92,8 +92,7 @@ int deviceCus() {
 // 1024 x 4096 25.4 -> 15.9; 128x128x64 s2 1024^3 11.7 -> 5.6; 128x64x64 s3 512^3 4.9 ->
 // 3.8; 64x128x128 s3 persistent 8192 x 128 x 4096 (128 tiles) 19.7 -> 15.3; 256x256x64
 // s2 1024 x 2048 x 1024 24.9 -> 7.7.
-template <int BM, int BN>
-int smallGridPart(int M, int N, int K) {
+int smallGridPart(int BM, int BN, int M, int N, int K) {
     if (BM * BN <= 64 * 64 || !ridge::partsFit(N, K)) return 0;
     const int cus = deviceCus();
     if ((M / BM) * (N / BN) > cus / 2) return 0;
@@ -104,30 +103,23 @@ int smallGridPart(int M, int N, int K) {
 }
 
 template <int PART>
-struct PartGrid {
-    ridge::TileOrder order;
-    dim3 grid;
-    PartGrid(int M, int N) {
-        using P = typename ridge::SmallGridPart<PART>::Part;
-        order = ridge::tileOrder<P::kBM, P::kBN, ridge::kPartGroupM>(M, N);
-        grid = dim3((unsigned)((M / P::kBM) * (N / P::kBN)));
-    }
-};
-
-template <int BM, int BN, int BK, int WM, int WN, int S, int G, int PART>
-void enqueuePersistentParts(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
-                            hipStream_t stream) {
-    const PartGrid<PART> g(M, N);
-    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, PART>), g.grid,
-                       dim3(ridge::kPartThreads), 0, stream, A, B, C, M, N, K, g.order.group, g.order.lastRows, 0u, 0,
-                       0, 0);
+void enqueuePart(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
+    using P = typename ridge::SmallGridPart<PART>::Part;
+    const ridge::TileOrder order = ridge::tileOrder<P::kBM, P::kBN, ridge::kPartGroupM>(M, N);
+    hipLaunchKernelGGL((ridge::gemmMfmaSmallGridKernel<PART>), dim3((unsigned)((M / P::kBM) * (N / P::kBN))),
+                       dim3(ridge::kPartThreads), 0, stream, A, B, C, M, N, K, order.group, order.lastRows);
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int S, int G, int PART>
-void enqueueUniformParts(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
-    const PartGrid<PART> g(M, N);
-    hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, false, PART>), g.grid,
-                       dim3(ridge::kPartThreads), 0, stream, A, B, C, M, N, K, g.order.group, g.order.lastRows, 0u);
+// Enqueues a small grid of a row's BM x BN tiles in its blocks; false where the row
+// runs its own tile.
+bool enqueueSmallGrid(int BM, int BN, const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
+                      hipStream_t stream) {
+    switch (smallGridPart(BM, BN, M, N, K)) {
+        case 1: enqueuePart<1>(A, B, C, M, N, K, stream); return true;
+        case 2: enqueuePart<2>(A, B, C, M, N, K, stream); return true;
+        case 3: enqueuePart<3>(A, B, C, M, N, K, stream); return true;
+        default: return false;
+    }
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
@@ -136,27 +128,11 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
     const auto* a = static_cast<const _Float16*>(A);
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
-    const int part = smallGridPart<BM, BN>(M, N, K);
-    if (part == 1) {
-        enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 1>(a, b, c, M, N, K, stream);
-        return hipGetLastError();
-    }
-    if constexpr (BN >= 128) {
-        if (part == 2) {
-            enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 2>(a, b, c, M, N, K, stream);
-            return hipGetLastError();
-        }
-    }
-    if constexpr (BM >= 128 && BN >= 128) {
-        if (part == 3) {
-            enqueuePersistentParts<BM, BN, BK, WM, WN, S, G, 3>(a, b, c, M, N, K, stream);
-            return hipGetLastError();
-        }
-    }
+    if (enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
     static SlotCache cache;
     hipError_t err;
     const int resident = cache.of(
-        reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, 0>), P::kThreads,
+        reinterpret_cast<const void*>(&ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), P::kThreads,
         &err);
     if (resident <= 0) return err;
     // Every workgroup must own at least one tile (the kernel's tile count per
@@ -164,7 +140,7 @@ hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N,
     const int tiles = (M / BM) * (N / BN);
     const int grid = tiles < resident ? tiles : resident;
     const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
-    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G, 0>), dim3((unsigned)grid),
+    hipLaunchKernelGGL((ridge::gemmMfmaPersistentKernel<BM, BN, BK, WM, WN, S, G>), dim3((unsigned)grid),
                        dim3(P::kThreads), 0, stream, a, b, c, M, N, K, order.group,
                        order.lastRows, ridge::reciprocalOf(K / BK), grid, tiles / grid, tiles % grid);
     return hipGetLastError();
@@ -231,26 +207,7 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
                            order.lastRows, whole, partTiles,
                            parts | phaseWidth(whole, slots, K) << 8);
     } else {
-        if constexpr (!NT && BM * BN > 64 * 64) {
-            const int part = smallGridPart<BM, BN>(M, N, K);
-            if (part == 1) {
-                enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 1>(A, B, C, M, N, K, stream);
-                return hipGetLastError();
-            }
-            if constexpr (BN >= 128) {
-                if (part == 2) {
-                    enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 2>(A, B, C, M, N, K, stream);
-                    return hipGetLastError();
-                }
-            }
-            if constexpr (BM >= 128 && BN >= 128) {
-                if (part == 3) {
-                    enqueueUniformParts<BM, BN, BK, WM, WN, S, G, 3>(A, B, C, M, N, K, stream);
-                    return hipGetLastError();
-                }
-            }
-        }
-        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT, 0>), dim3((unsigned)tiles), block, 0,
+        hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
                            stream, A, B, C, M, N, K, order.group, order.lastRows, ridge::reciprocalOf(K / BK));
     }
     return hipGetLastError();
@@ -262,6 +219,7 @@ hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, in
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
     constexpr bool pingPong = usesPingPong(ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kWaves, S);
+    if (!pingPong && enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
     if ((size_t)M * N * 2 > ridge::kNonTemporalBytes && !(pingPong && K < ridge::kNonTemporalPingPongK))
         return enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
     return enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);

@@ -677,8 +677,9 @@ using Part128x128 = TilePart<128, 128, 32, 64, 3>;
 using Part64x128 = TilePart<64, 128, 32, 32, 3>;
 using Part64x64 = TilePart<64, 64, 16, 32, 4>;
 
-// Kernels that carry a row's template arguments run a whole small grid in blocks of
-// PART (smallGridPart in gemm_kernels.hip): 0 is the row's own tile.
+// The blocks in which uniform and persistent rows run a whole small grid (smallGridPart
+// in gemm_kernels.hip), by number. One kernel per block: its code does not depend on
+// the row.
 template <int PART>
 struct SmallGridPart;
 template <>
@@ -697,53 +698,52 @@ constexpr int kPartThreads = 512;
 constexpr int kPartGroupM = 8;
 
 template <int PART>
-__device__ __forceinline__ void runSmallGrid(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
-                                             TileOrder order) {
+__global__ __launch_bounds__(kPartThreads)
+void gemmMfmaSmallGridKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
+                             _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
+                             uint32_t lastRowsReciprocal) {
     using P = typename SmallGridPart<PART>::Part;
     static_assert(P::Blk::T::kThreads == kPartThreads, "parts have eight wavefronts");
     __shared__ __attribute__((aligned(1024))) char lds[P::Blk::T::kLdsBytes];
     int row, col;
     const int tiles = (M / P::kBM) * (N / P::kBN);
-    tileOf<P::kBM, P::kBN, kPartGroupM>(xcdRemap(blockIdx.x, tiles), M, N, order, row, col);
+    tileOf<P::kBM, P::kBN, kPartGroupM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row,
+                                        col);
     P::template run<false>(lds, A, B, C, row, col, N, K);
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT, int PART>
-__global__ __launch_bounds__(PART != 0 ? kPartThreads : (BM / WM) * (BN / WN) * kWaveSize)
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, bool NT>
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * kWaveSize)
 void gemmMfmaKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                     _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
                     uint32_t lastRowsReciprocal, uint32_t numKReciprocal) {
-    if constexpr (PART != 0) {
-        runSmallGrid<PART>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal});
-    } else {
-        using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
-        __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
-        int row, col;
-        const int tiles = (M / BM) * (N / BN);  // = gridDim.x, which would be a load
-        tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
-        GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
-        const int numK = K / BK;
-        // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
-        // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
-        // Cold, when the first touch of every K slice comes from HBM, workgroups in
-        // lockstep all request the same K slice of their panels at once (A's slice
-        // strided by a row); staggered, they request different slices. Measured at
-        // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
-        // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
-        // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
-        // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
-        // long K loops, which gained nothing. Only the summation order of the K tiles
-        // changes.
-        constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
-        if constexpr (kStagger) {
-            if (numK <= 32) blk.kStart = (int)divide((uint32_t)(row / BM + col / BN), numK, numKReciprocal).rem;
-        }
-
-        // The 8-wave rows (two stages, 256 registers per lane) keep the general form
-        // of the loop only: the second copy made them spill.
-        uniformLoop<kStagger, (T::kWaves <= 4)>(blk, numK);
-        blk.template store<NT>(C, N);
+    using T = GemmTraits<BM, BN, BK, WM, WN, STAGES, GROUPM>;
+    __shared__ __attribute__((aligned(1024))) char lds[T::kLdsBytes];
+    int row, col;
+    const int tiles = (M / BM) * (N / BN);  // = gridDim.x, which would be a load
+    tileOf<BM, BN, GROUPM>(xcdRemap(blockIdx.x, tiles), M, N, {groupReciprocal, lastRowsReciprocal}, row, col);
+    GemmBlock<BM, BN, BK, WM, WN, STAGES, GROUPM> blk(lds, A, B, row, col, N, K);
+    const int numK = K / BK;
+    // K stagger for the short K loops of 4-wave BK >= 64 rows: each workgroup
+    // starts its K loop at K tile (tile row + tile column) mod K/BK and wraps.
+    // Cold, when the first touch of every K slice comes from HBM, workgroups in
+    // lockstep all request the same K slice of their panels at once (A's slice
+    // strided by a row); staggered, they request different slices. Measured at
+    // 1024^3 and 2048 x 2048 x 1024: 5-16% faster cold, between 1.6% slower and
+    // 3% faster warm. Not taken where it measured worse: BK = 32 rows (up to 6%
+    // slower warm), 8-wave rows (256 x 256 x 64 s2 2% slower at 4096 x 4096 x
+    // 2048, whose panels outgrow the L2 once the workgroups drift apart), and
+    // long K loops, which gained nothing. Only the summation order of the K tiles
+    // changes.
+    constexpr bool kStagger = BK >= 64 && T::kWaves <= 4;
+    if constexpr (kStagger) {
+        if (numK <= 32) blk.kStart = (int)divide((uint32_t)(row / BM + col / BN), numK, numKReciprocal).rem;
     }
+
+    // The 8-wave rows (two stages, 256 registers per lane) keep the general form
+    // of the loop only: the second copy made them spill.
+    uniformLoop<kStagger, (T::kWaves <= 4)>(blk, numK);
+    blk.template store<NT>(C, N);
 }
 
 // ---------------------------------------------------------------------------
@@ -1175,18 +1175,14 @@ __device__ __forceinline__ void persistentWalk(const _Float16* A, const _Float16
     for (; g0 < G; g0 += U) pass(g0, std::false_type{});
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM, int PART>
-__global__ __launch_bounds__(PART != 0 ? kPartThreads : ((BM / WM) * (BN / WN) + kPersistentLoaders) * kWaveSize)
+template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUPM>
+__global__ __launch_bounds__(((BM / WM) * (BN / WN) + kPersistentLoaders) * kWaveSize)
 void gemmMfmaPersistentKernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                               _Float16* __restrict__ C, int M, int N, int K, uint32_t groupReciprocal,
                               uint32_t lastRowsReciprocal, uint32_t numKReciprocal, int grid, int tilesEach,
                               int tilesMore) {
-    if constexpr (PART != 0) {
-        runSmallGrid<PART>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal});
-    } else {
-        persistentWalk<BM, BN, BK, WM, WN, STAGES, GROUPM>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal},
-                                                           numKReciprocal, grid, tilesEach, tilesMore);
-    }
+    persistentWalk<BM, BN, BK, WM, WN, STAGES, GROUPM>(A, B, C, M, N, K, {groupReciprocal, lastRowsReciprocal},
+                                                       numKReciprocal, grid, tilesEach, tilesMore);
 }
 
 }  // namespace ridge

@@ -415,9 +415,9 @@ def cmd_run(args):
 
 # Kernel names as rocprofv3 reports them: Itanium-mangled, each int template
 # argument as Li<n>E (gemmMfmaKernelILi64ELi64E...), or demangled (<64, 64, ...>);
-# a bool (non-temporal stores) and an int (small-grid blocks) may follow the seven.
+# a bool (non-temporal stores) may follow the seven.
 _GEMM_NAME = re.compile(r"gemmMfma(?:PingPong|Persistent)?Kernel(?:I" + r"Li(\d+)E" * 7 + r"|<" +
-                        r",".join([r"\s*(\d+)"] * 7) + r"\s*(?:,\s*(?:true|false|\d+)\s*)*>)")
+                        r",".join([r"\s*(\d+)"] * 7) + r"\s*(?:,\s*(?:true|false)\s*)?>)")
 
 
 def _template_args(name):

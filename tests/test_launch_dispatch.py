@@ -42,7 +42,7 @@ int hipLaunchKernel(const void* fn, dim3_t g, dim3_t b, void** args, size_t n, v
     (void)n; (void)s;
     for (int i = 0; i < count; ++i)
         if (kernels[i].fn == fn) name = kernels[i].name;
-    const int ints = strstr(name, "PingPong") ? 8 : strstr(name, "Persistent") ? 9 : 6;
+    const int ints = strstr(name, "PingPong") ? 8 : strstr(name, "Persistent") ? 9 : strstr(name, "Small") ? 5 : 6;
     printf("{\"kernel\": \"%s\", \"grid\": %u, \"block\": %u, \"args\": [", name, g.x, b.x);
     for (int i = 0; i < ints; ++i) printf("%s%u", i ? ", " : "", *(uint32_t*)args[3 + i]);
     printf("]}\n");
@@ -160,3 +160,24 @@ def test_a_launch_whose_device_query_fails_runs_its_own_tiles_and_succeeds(fake_
         if query != "hipOccupancy":
             assert made[0]["grid"] == (M // v.BM) * (N // v.BN), v.label()
             assert made[0]["block"] == v.threads, v.label()
+
+
+@pytest.mark.parametrize("M,N,K,block", [(1024, 1024, 128, (64, 64)), (2048, 1024, 128, (64, 128)),
+                                         (2048, 2048, 128, (128, 128)), (4096, 4096, 128, None),
+                                         (1024, 1024, 96, None)])
+def test_small_grids_run_one_kernel_per_block_whatever_the_row(fake_hip, M, N, K, block):
+    """A uniform or persistent row's grid of at most 128 tiles on 256 CUs, in the
+    smallest block whose workgroups fit one round: the same kernel for every row."""
+    names = {}
+    picked = [v for v in rows(0) + rows(2) if v.divides(M, N, K) and (v.BM, v.BN) != (64, 64)]
+    for v, (rc, made) in zip(picked, launches(fake_hip, [(v.index, M, N, K) for v in picked])):
+        assert rc == 0 and len(made) == 1
+        tiles = (M // v.BM) * (N // v.BN)
+        small = "SmallGrid" in made[0]["kernel"]
+        assert small == (tiles <= 128 and block is not None), v.label()
+        if small:
+            assert made[0]["grid"] == (M // block[0]) * (N // block[1]), v.label()
+            names.setdefault(made[0]["kernel"], []).append(v.index)
+        elif v.schedule == 0:
+            assert made[0]["grid"] == tiles, v.label()
+    assert len(names) == (1 if block else 0), names
