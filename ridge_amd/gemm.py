@@ -176,13 +176,29 @@ def _ptr(x):
     return x.data_ptr()
 
 
+_raw_calls = None
+
+
+def _current():
+    """(call for the current device's index, call from an index to that device's current
+    stream handle). torch's own raw calls where it has them: no Stream object is built
+    (2.8 -> 0.5 us, of a launch that costs 4). They are not part of its public interface,
+    so a torch without one gets the public call."""
+    global _raw_calls
+    if _raw_calls is None:
+        import torch
+        _raw_calls = (getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device),
+                      getattr(torch._C, "_cuda_getCurrentRawStream",
+                              lambda device: torch.cuda.current_stream(device).cuda_stream))
+    return _raw_calls
+
+
 def _stream_handle(stream):
     if stream is None:
         import torch
         if torch.cuda.is_initialized():
-            # The same handle without building a Stream object (2.8 -> 0.5 us, of a
-            # launch that costs 4).
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+            device, handle = _raw_calls or _current()
+            return handle(device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
@@ -269,7 +285,7 @@ def gemm(A, B, index=0, out=None, stream=None):
     N = B.shape[1]
     C = out if out is not None else torch.empty((M, N), dtype=torch.float16, device=A.device)
     # The library launches on the current device; make it the operands' one.
-    if torch._C._cuda_getDevice() == A.device.index:
+    if (_raw_calls or _current())[0]() == A.device.index:
         rc = launch(index, A, B, C, M, N, K, stream)
     else:
         with torch.cuda.device(A.device):

@@ -181,3 +181,21 @@ def test_small_grids_run_one_kernel_per_block_whatever_the_row(fake_hip, M, N, K
         elif v.schedule == 0:
             assert made[0]["grid"] == tiles, v.label()
     assert len(names) == (1 if block else 0), names
+
+
+@pytest.mark.parametrize("absent", ["_cuda_getDevice", "_cuda_getCurrentRawStream"])
+def test_the_current_stream_without_torchs_raw_calls(monkeypatch, absent):
+    """A torch that lacks one of the raw calls: the public ones give the same handle."""
+    torch = pytest.importorskip("torch")
+
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream if device == 3 else None)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 3)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 77 if device == 3 else None)
+    monkeypatch.delattr(torch._C, absent)
+    monkeypatch.setattr(G, "_raw_calls", None, raising=False)
+    assert G._stream_handle(None) == 77
