@@ -79,8 +79,29 @@ int ridge_gemm_divides(int i, int M, int N, int K);
  * the launch error. The reference's KernelVariant::launch (gemm-mma.cu:19-43).
  * Where the row's tiles would leave most CUs idle (a small grid, or the last partial
  * round of a ping-pong row) they run in smaller blocks of 512 threads within the same
- * launch; the row's fields describe its own tile. */
+ * launch; the row's fields describe its own tile. ridge_gemm_launch_form says which. */
 int ridge_gemm_launch(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
+
+/* ridge_gemm_launch with the row's own tile over the whole grid, however few tiles there
+ * are: the kernel that the row's fields, the cost model and the sweeps describe. For
+ * measuring a row and for tests; a small grid runs up to several times longer. */
+int ridge_gemm_launch_own_tile(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream);
+
+/* How ridge_gemm_launch runs M x N x K with variant i on a device of numCUs CUs: ownTiles
+ * output tiles in the row's own tile, and what is left (nothing: partWorkgroups is 0 and
+ * so are the other fields) in partWorkgroups workgroups of a partBM x partBN x partBK
+ * block on wavefront tiles of partWM x partWN and a ring of partStages. A uniform or
+ * persistent row runs all of its grid one way; a ping-pong row's last round may be parts.
+ * No device is touched. Returns 0, or 1 (hipErrorInvalidValue) for a bad index, a shape
+ * that the row does not divide, a null pointer or numCUs below 1. */
+typedef struct ridge_gemm_form {
+    int ownTiles;
+    int partWorkgroups;
+    int partBM, partBN, partBK;
+    int partWM, partWN;
+    int partStages;
+} ridge_gemm_form_t;
+int ridge_gemm_launch_form(int i, int M, int N, int K, int numCUs, ridge_gemm_form_t* out);
 
 /* Writes the variant table as CSV (header then one row per variant) into buf.
  * Returns the number of bytes the full text needs (excluding the NUL); writes at

@@ -18,7 +18,17 @@
 
 namespace {
 
-typedef hipError_t (*LaunchFn)(const void*, const void*, void*, int, int, int, hipStream_t);
+// How a launch runs a row's output tiles: ownTiles of them in the row's own tile and the
+// others in partWorkgroups blocks of `part`, as parts of tiles (a ping-pong row's last
+// round) or as the whole grid's blocks (smallGrid, a number of ridge::SmallGridPart).
+struct Form {
+    int ownTiles = 0, parts = 1, smallGrid = 0, partWorkgroups = 0;
+    ridge::BlockShape part = {};
+};
+
+// With ownTile the row's tile runs everywhere, whatever the grid.
+typedef hipError_t (*LaunchFn)(const void*, const void*, void*, int, int, int, bool ownTile, hipStream_t);
+typedef Form (*FormFn)(int M, int N, int K, int cus);
 
 // Schedules (ridge_gemm_variant_t.schedule). Rows written RIDGE_VARIANT take
 // theirs from the tile config: eight wavefronts (two per SIMD) with a ring of
@@ -92,9 +102,8 @@ int deviceCus() {
 // 1024 x 4096 25.4 -> 15.9; 128x128x64 s2 1024^3 11.7 -> 5.6; 128x64x64 s3 512^3 4.9 ->
 // 3.8; 64x128x128 s3 persistent 8192 x 128 x 4096 (128 tiles) 19.7 -> 15.3; 256x256x64
 // s2 1024 x 2048 x 1024 24.9 -> 7.7.
-int smallGridPart(int BM, int BN, int M, int N, int K) {
+int smallGridPart(int BM, int BN, int M, int N, int K, int cus) {
     if (BM * BN <= 64 * 64 || !ridge::partsFit(N, K)) return 0;
-    const int cus = deviceCus();
     if ((M / BM) * (N / BN) > cus / 2) return 0;
     if ((M / 64) * (N / 64) <= cus) return 1;
     if (BN >= 128 && (M / 64) * (N / 128) <= cus) return 2;
@@ -114,7 +123,8 @@ void enqueuePart(const _Float16* A, const _Float16* B, _Float16* C, int M, int N
 // runs its own tile.
 bool enqueueSmallGrid(int BM, int BN, const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K,
                       hipStream_t stream) {
-    switch (smallGridPart(BM, BN, M, N, K)) {
+    if (BM * BN <= 64 * 64) return false;
+    switch (smallGridPart(BM, BN, M, N, K, deviceCus())) {
         case 1: enqueuePart<1>(A, B, C, M, N, K, stream); return true;
         case 2: enqueuePart<2>(A, B, C, M, N, K, stream); return true;
         case 3: enqueuePart<3>(A, B, C, M, N, K, stream); return true;
@@ -122,13 +132,28 @@ bool enqueueSmallGrid(int BM, int BN, const _Float16* A, const _Float16* B, _Flo
     }
 }
 
+Form smallGridForm(int BM, int BN, int M, int N, int K, int cus) {
+    Form f;
+    f.smallGrid = smallGridPart(BM, BN, M, N, K, cus);
+    if (f.smallGrid == 0) {
+        f.ownTiles = (M / BM) * (N / BN);
+        return f;
+    }
+    f.part = f.smallGrid == 1   ? ridge::SmallGridPart<1>::Part::kShape
+             : f.smallGrid == 2 ? ridge::SmallGridPart<2>::Part::kShape
+                                : ridge::SmallGridPart<3>::Part::kShape;
+    f.partWorkgroups = (M / f.part.BM) * (N / f.part.BN);
+    return f;
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
-hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
+hipError_t launchPersistent(const void* A, const void* B, void* C, int M, int N, int K, bool ownTile,
+                            hipStream_t stream) {
     using P = ridge::PersistentTraits<BM, BN, BK, WM, WN, S, G>;
     const auto* a = static_cast<const _Float16*>(A);
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
-    if (enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
+    if (!ownTile && enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
     static SlotCache cache;
     hipError_t err;
     const int resident = cache.of(
@@ -188,24 +213,35 @@ int phaseWidth(int wholeTiles, int slots, int K) {
     return slots >= ridge::kPhases && wholeTiles / slots >= 3 && K <= 2048 ? slots / ridge::kPhases : 0;
 }
 
+template <int BM, int BN, int BK>
+Form pingPongForm(int M, int N, int K, int cus) {
+    using Tail = ridge::TailTiles<BM, BN, BK>;
+    const int tiles = (M / BM) * (N / BN);
+    // A device that does not say its CUs runs every tile whole.
+    const int rem = cus > 0 ? tiles % cus : 0;
+    Form f;
+    f.parts = tailParts(rem, cus, N, K, Tail::kParts);
+    f.ownTiles = f.parts > 1 ? tiles - rem : tiles;
+    f.partWorkgroups = (tiles - f.ownTiles) * f.parts;
+    if (f.parts > 1) f.part = Tail::shapeOf(f.parts);
+    return f;
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, int G, bool NT>
-hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, hipStream_t stream) {
+hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M, int N, int K, bool ownTile,
+                        hipStream_t stream) {
     using T = ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>;
     const int tiles = (M / BM) * (N / BN);
     const dim3 block(T::kThreads);
     const ridge::TileOrder order = ridge::tileOrder<BM, BN, G>(M, N);
     if constexpr (usesPingPong(T::kWaves, S)) {
         static_assert(2 * T::kLdsBytes > 163840, "a ping-pong row has one workgroup per CU");
-        const int slots = deviceCus();
-        // A device that does not say its CUs runs every tile whole.
-        const int rem = slots > 0 ? tiles % slots : 0;
-        const int parts = tailParts(rem, slots, N, K, ridge::TailTiles<BM, BN, BK>::kParts);
-        const int whole = parts > 1 ? tiles - rem : tiles;
-        const int partTiles = (tiles - whole) * parts;
+        const int cus = deviceCus();
+        const Form f = pingPongForm<BM, BN, BK>(M, N, K, ownTile ? 0 : cus);
         hipLaunchKernelGGL((ridge::gemmMfmaPingPongKernel<BM, BN, BK, WM, WN, S, G, NT>),
-                           dim3((unsigned)(whole + partTiles)), block, 0, stream, A, B, C, M, N, K, order.group,
-                           order.lastRows, whole, partTiles,
-                           parts | phaseWidth(whole, slots, K) << 8);
+                           dim3((unsigned)(f.ownTiles + f.partWorkgroups)), block, 0, stream, A, B, C, M, N, K,
+                           order.group, order.lastRows, f.ownTiles, f.partWorkgroups,
+                           f.parts | phaseWidth(f.ownTiles, cus, K) << 8);
     } else {
         hipLaunchKernelGGL((ridge::gemmMfmaKernel<BM, BN, BK, WM, WN, S, G, NT>), dim3((unsigned)tiles), block, 0,
                            stream, A, B, C, M, N, K, order.group, order.lastRows, ridge::reciprocalOf(K / BK));
@@ -214,15 +250,27 @@ hipError_t enqueueTiles(const _Float16* A, const _Float16* B, _Float16* C, int M
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int S, int G>
-hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
+hipError_t launchVariant(const void* A, const void* B, void* C, int M, int N, int K, bool ownTile,
+                         hipStream_t stream) {
     const auto* a = static_cast<const _Float16*>(A);
     const auto* b = static_cast<const _Float16*>(B);
     auto* c = static_cast<_Float16*>(C);
     constexpr bool pingPong = usesPingPong(ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kWaves, S);
-    if (!pingPong && enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
+    if (!pingPong && !ownTile && enqueueSmallGrid(BM, BN, a, b, c, M, N, K, stream)) return hipGetLastError();
     if ((size_t)M * N * 2 > ridge::kNonTemporalBytes && !(pingPong && K < ridge::kNonTemporalPingPongK))
-        return enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, stream);
-    return enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, stream);
+        return enqueueTiles<BM, BN, BK, WM, WN, S, G, true>(a, b, c, M, N, K, ownTile, stream);
+    return enqueueTiles<BM, BN, BK, WM, WN, S, G, false>(a, b, c, M, N, K, ownTile, stream);
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int S>
+Form formOf(int M, int N, int K, int cus) {
+    if constexpr (usesPingPong((BM / WM) * (BN / WN), S)) return pingPongForm<BM, BN, BK>(M, N, K, cus);
+    return smallGridForm(BM, BN, M, N, K, cus);
+}
+
+template <int BM, int BN>
+Form formOfPersistent(int M, int N, int K, int cus) {
+    return smallGridForm(BM, BN, M, N, K, cus);
 }
 
 struct Entry {
@@ -232,6 +280,7 @@ struct Entry {
     int waves;
     int schedule;
     LaunchFn launch;
+    FormFn form;
 };
 
 #define RIDGE_VARIANT(BM, BN, BK, WM, WN, S, G)                                              \
@@ -240,7 +289,8 @@ struct Entry {
           ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kThreads,                             \
           ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kWaves,                               \
           usesPingPong(ridge::GemmTraits<BM, BN, BK, WM, WN, S, G>::kWaves, S) ? kPingPong : kUniform, \
-          &launchVariant<BM, BN, BK, WM, WN, S, G>},
+          &launchVariant<BM, BN, BK, WM, WN, S, G>,                                          \
+          &formOf<BM, BN, BK, WM, WN, S>},
 
 // ldsBytes includes the epilogue staging; threads and waves include the two
 // loader wavefronts.
@@ -250,7 +300,8 @@ struct Entry {
           ridge::PersistentTraits<BM, BN, BK, WM, WN, S, G>::kThreads,                       \
           ridge::PersistentTraits<BM, BN, BK, WM, WN, S, G>::kWaves,                         \
           kPersistent,                                                                       \
-          &launchPersistent<BM, BN, BK, WM, WN, S, G>},
+          &launchPersistent<BM, BN, BK, WM, WN, S, G>,                                       \
+          &formOfPersistent<BM, BN>},
 
 const Entry kTable[] = {
 #include "gemm_variants.def"
@@ -311,11 +362,30 @@ int ridge_gemm_divides(int i, int M, int N, int K) {
     return ridge::tileOffsetsFit(e.BM, e.BK, N, K) ? 1 : 0;
 }
 
-int ridge_gemm_launch(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream) {
+static int launchRow(int i, const void* A, const void* B, void* C, int M, int N, int K, bool ownTile,
+                     void* stream) {
     if (!ridge_gemm_divides(i, M, N, K)) return (int)hipErrorInvalidValue;
     if (A == nullptr || B == nullptr || C == nullptr) return (int)hipErrorInvalidValue;
     if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15u) return (int)hipErrorInvalidValue;
-    return (int)kTable[i].launch(A, B, C, M, N, K, static_cast<hipStream_t>(stream));
+    return (int)kTable[i].launch(A, B, C, M, N, K, ownTile, static_cast<hipStream_t>(stream));
+}
+
+int ridge_gemm_launch(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream) {
+    return launchRow(i, A, B, C, M, N, K, false, stream);
+}
+
+int ridge_gemm_launch_own_tile(int i, const void* A, const void* B, void* C, int M, int N, int K, void* stream) {
+    return launchRow(i, A, B, C, M, N, K, true, stream);
+}
+
+int ridge_gemm_launch_form(int i, int M, int N, int K, int numCUs, ridge_gemm_form_t* out) {
+    if (out == nullptr || numCUs <= 0 || !ridge_gemm_divides(i, M, N, K)) return (int)hipErrorInvalidValue;
+    const Form f = kTable[i].form(M, N, K, numCUs);
+    out->ownTiles = f.ownTiles;
+    out->partWorkgroups = f.partWorkgroups;
+    out->partBM = f.part.BM; out->partBN = f.part.BN; out->partBK = f.part.BK;
+    out->partWM = f.part.WM; out->partWN = f.part.WN; out->partStages = f.part.stages;
+    return 0;
 }
 
 int ridge_gemm_split_rows(int body, int M, int N, int K, int numCUs) {

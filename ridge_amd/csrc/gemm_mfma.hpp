@@ -660,8 +660,13 @@ constexpr bool partsFit(int N, int K) {
     return K % kPartBK == 0 && tileOffsetsFit(kPartMostBM, kPartBK, N, K);
 }
 
+struct BlockShape {
+    int BM, BN, BK, WM, WN, stages;
+};
+
 template <int BM, int BN, int WM, int WN, int STAGES>
 struct TilePart {
+    static constexpr BlockShape kShape = {BM, BN, kPartBK, WM, WN, STAGES};
     static_assert(BM <= kPartMostBM, "partsFit bounds the offsets of blocks of at most this many rows");
     static constexpr int kBM = BM, kBN = BN;
     using Blk = GemmBlock<BM, BN, kPartBK, WM, WN, STAGES, 1>;
@@ -862,6 +867,7 @@ template <int BM, int BN, int BK>
 struct TailTiles {
     static constexpr int kParts = 1;      // the most parts of one tile
     static constexpr int kLdsBytes = 0;
+    static constexpr BlockShape shapeOf(int) { return {}; }   // the block of each of `parts` parts
 };
 
 template <>
@@ -871,6 +877,12 @@ struct TailTiles<256, 256, 32> {
     static constexpr int kLdsBytes = Part128x128::Blk::T::kLdsBytes;
     static_assert(Half::T::kLdsBytes <= kLdsBytes && Part64x128::Blk::T::kLdsBytes <= kLdsBytes &&
                   Part64x64::Blk::T::kLdsBytes <= kLdsBytes, "the quarters need the most LDS");
+    static constexpr BlockShape shapeOf(int parts) {
+        return parts == 16  ? Part64x64::kShape
+               : parts == 8 ? Part64x128::kShape
+               : parts == 4 ? Part128x128::kShape
+                            : BlockShape{128, 256, 32, 64, 64, 3};
+    }
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int part, int parts, int N, int K) {
@@ -892,6 +904,9 @@ template <>
 struct TailTiles<256, 128, 64> {
     static constexpr int kParts = 8;
     static constexpr int kLdsBytes = Part128x128::Blk::T::kLdsBytes;
+    static constexpr BlockShape shapeOf(int parts) {
+        return parts == 8 ? Part64x64::kShape : parts == 4 ? Part64x128::kShape : Part128x128::kShape;
+    }
     template <bool NT>
     static __device__ __forceinline__ void run(const char* lds, const _Float16* A, const _Float16* B, _Float16* C,
                                                int row, int col, int part, int parts, int N, int K) {

@@ -10,6 +10,8 @@ exposes the same surface in Python:
     variant(i)                 -> Variant
     find_variant(BM, BN, ...)  -> index or -1
     launch(i, A, B, C, M, N, K, stream) -> hipError_t value (0 = success)
+    launch_form(i, M, N, K)    -> Form (which blocks such a launch runs)
+    launch_own_tile(i, ...)    -> launch() in the row's own tile, whatever the grid
     gemm(A, B, i)              -> C, raising on any error
 
 Device buffers are torch tensors (or raw device addresses); torch provides device
@@ -38,6 +40,12 @@ class _VariantStruct(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int) for n in (
         "BM", "BN", "BK", "WM", "WN", "stages", "groupM", "ldsBytes", "threads", "regsPerThread",
         "waves", "vgprs", "agprs", "sgprs", "scratchBytes", "occupancy", "pingPong", "schedule")]
+
+
+class _FormStruct(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in (
+        "ownTiles", "partWorkgroups", "partBM", "partBN", "partBK", "partWM", "partWN", "partStages")]
+
 
 SCHEDULES = {0: "uniform", 1: "ping-pong", 2: "persistent"}
 
@@ -88,6 +96,24 @@ class Variant:
         return asdict(self)
 
 
+@dataclass(frozen=True)
+class Form:
+    """How a launch runs (ridge_gemm_launch_form): ownTiles output tiles in the row's own
+    tile, the rest in partWorkgroups blocks of part* (all 0 where there is no rest)."""
+    ownTiles: int
+    partWorkgroups: int
+    partBM: int
+    partBN: int
+    partBK: int
+    partWM: int
+    partWN: int
+    partStages: int
+
+    @property
+    def own(self):
+        return self.partWorkgroups == 0
+
+
 def lib():
     """Loads libridge_gemm.so once. Raises if it has not been built."""
     global _lib
@@ -108,6 +134,10 @@ def lib():
     L.ridge_gemm_divides.argtypes = [c_int] * 4
     L.ridge_gemm_launch.restype = c_int
     L.ridge_gemm_launch.argtypes = [c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
+    L.ridge_gemm_launch_own_tile.restype = c_int
+    L.ridge_gemm_launch_own_tile.argtypes = L.ridge_gemm_launch.argtypes
+    L.ridge_gemm_launch_form.restype = c_int
+    L.ridge_gemm_launch_form.argtypes = [c_int] * 5 + [ctypes.POINTER(_FormStruct)]
     L.ridge_gemm_split_rows.restype = c_int
     L.ridge_gemm_split_rows.argtypes = [c_int] * 5
     L.ridge_gemm_launch_split.restype = c_int
@@ -208,6 +238,20 @@ def _stream_handle(stream):
 def launch(i, A, B, C, M, N, K, stream=None):
     """Enqueues C = A B with variant i; returns the hipError_t value."""
     return lib().ridge_gemm_launch(i, _ptr(A), _ptr(B), _ptr(C), M, N, K, _stream_handle(stream))
+
+
+def launch_own_tile(i, A, B, C, M, N, K, stream=None):
+    """launch() in the row's own tile over the whole grid, for measuring a row."""
+    return lib().ridge_gemm_launch_own_tile(i, _ptr(A), _ptr(B), _ptr(C), M, N, K, _stream_handle(stream))
+
+
+def launch_form(i, M, N, K, num_cus=256):
+    """How launch() runs M x N x K with variant i on a device of num_cus CUs."""
+    s = _FormStruct()
+    rc = lib().ridge_gemm_launch_form(i, M, N, K, num_cus, ctypes.byref(s))
+    if rc != HIP_SUCCESS:
+        raise RidgeGemmError("variant %d has no launch of %dx%dx%d on %d CUs" % (i, M, N, K, num_cus))
+    return Form(*[getattr(s, f) for f, _ in _FormStruct._fields_])
 
 
 def bound_launch(i, A, B, C, M, N, K, stream=None):

@@ -3,6 +3,7 @@ runs in a child process on a stand-in for the HIP runtime, which records the lau
 instead of making them and can be told to refuse a device query."""
 import json
 import os
+import random
 import subprocess
 import sys
 
@@ -76,9 +77,10 @@ CHILD = r"""
 import ctypes, json, sys
 ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 L = ctypes.CDLL(sys.argv[2])
-L.ridge_gemm_launch.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+launch = getattr(L, sys.argv[3])
+launch.argtypes = [ctypes.c_int] + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]
 for call in json.load(sys.stdin):
-    rc = L.ridge_gemm_launch(call[0], 4096, 4096, 4096, call[1], call[2], call[3], None)
+    rc = launch(call[0], 4096, 4096, 4096, call[1], call[2], call[3], None)
     print(json.dumps({"rc": rc}), flush=True)
 """
 
@@ -92,11 +94,11 @@ def fake_hip(tmp_path_factory):
     return str(so)
 
 
-def launches(fake_hip, calls, refuses=""):
+def launches(fake_hip, calls, refuses="", entry="ridge_gemm_launch"):
     """[(return code, the launches made)] of calls (variant index, M, N, K)."""
     env = dict(os.environ, FAKE_HIP_REFUSES=refuses)
-    p = subprocess.run([sys.executable, "-c", CHILD, fake_hip, G.LIB_PATH], input=json.dumps(calls), env=env,
-                       capture_output=True, text=True, timeout=120)
+    p = subprocess.run([sys.executable, "-c", CHILD, fake_hip, G.LIB_PATH, entry], input=json.dumps(calls),
+                       env=env, capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
     out, made = [], []
     for line in p.stdout.splitlines():
@@ -181,6 +183,68 @@ def test_small_grids_run_one_kernel_per_block_whatever_the_row(fake_hip, M, N, K
         elif v.schedule == 0:
             assert made[0]["grid"] == tiles, v.label()
     assert len(names) == (1 if block else 0), names
+
+
+def _form_shapes(v):
+    """Grids on every side of the rules on 256 CUs: tile counts around half a round and
+    around a sixteenth, an eighth, a quarter and a half of a round, alone and behind
+    whole rounds; K on and off the parts' 64; N beyond what their offsets hold."""
+    rng = random.Random(v.index)
+    counts = [1, 2, 3, 16, 17, 32, 33, 64, 65, 100, 127, 128, 129, 200, 256]
+    shapes = []
+    for n in counts + [256 + c for c in counts] + [1024 + c for c in counts]:
+        m = rng.choice([d for d in range(1, n + 1) if n % d == 0])
+        shapes.append((v.BM * m, v.BN * (n // m), v.BK * rng.choice([1, 2, 3, 8])))
+    shapes += [(v.BM, v.BN * (130816 + c), 64) for c in (1, 16, 33, 65, 129)]
+    shapes += [(v.BM, v.BN * (133120 + c), 64) for c in (1, 16, 33, 65, 129)]
+    return [s for s in shapes if v.divides(*s)]
+
+
+@pytest.mark.parametrize("schedule", [0, 1, 2])
+def test_launch_form_says_what_the_launch_runs(fake_hip, schedule):
+    picked = [(v, s) for v in rows(schedule) for s in _form_shapes(v)]
+    kinds = set()
+    for (v, (M, N, K)), (rc, made) in zip(picked, launches(fake_hip, [(v.index,) + s for v, s in picked])):
+        what = "%s on %dx%dx%d" % (v.label(), M, N, K)
+        assert rc == 0 and len(made) == 1, what
+        f, tiles = G.launch_form(v.index, M, N, K), (M // v.BM) * (N // v.BN)
+        # Every output once, in blocks that fit one round, the shape and 32-bit offsets.
+        assert f.ownTiles * v.BM * v.BN + f.partWorkgroups * f.partBM * f.partBN == M * N, what
+        assert f.own == (f.partBM == 0) == (f.ownTiles == tiles), what
+        if not f.own:
+            assert f.partWorkgroups <= 256 and K % f.partBK == 0, what
+            assert f.partBK * N < 2 ** 31 and f.partBM * K < 2 ** 31, what
+            assert (f.partBM // f.partWM) * (f.partBN // f.partWN) * 64 == 512, what
+        if schedule == 1:
+            whole, part_workgroups, parts = ping_pong_parts(made[0])
+            assert (whole, part_workgroups) == (f.ownTiles, f.partWorkgroups), what
+            assert made[0]["grid"] == whole + part_workgroups and tiles == whole + part_workgroups // parts, what
+        else:
+            assert f.own == ("SmallGrid" not in made[0]["kernel"]) and f.ownTiles in (0, tiles), what
+            want = f.partWorkgroups if not f.own else tiles if schedule == 0 else min(tiles, 256)
+            assert made[0]["grid"] == want, what
+        kinds.add((f.partBM, f.partBN, f.partBK))
+    assert len(kinds) == {0: 4, 1: 5, 2: 4}[schedule], kinds
+
+
+@pytest.mark.parametrize("schedule", [0, 1, 2])
+def test_launch_own_tile_runs_the_rows_tile_on_every_grid(fake_hip, schedule):
+    picked = [(v, s) for v in rows(schedule) for s in _form_shapes(v)]
+    calls = [(v.index,) + s for v, s in picked]
+    for (v, (M, N, K)), (rc, made) in zip(picked, launches(fake_hip, calls, entry="ridge_gemm_launch_own_tile")):
+        tiles = (M // v.BM) * (N // v.BN)
+        assert rc == 0 and len(made) == 1 and "SmallGrid" not in made[0]["kernel"]
+        assert made[0]["grid"] == (min(tiles, 256) if schedule == 2 else tiles)
+        assert made[0]["block"] == v.threads
+        if schedule == 1:
+            assert ping_pong_parts(made[0]) == (tiles, 0, 1)
+
+
+def test_launch_form_refuses_what_a_launch_refuses():
+    for args in ((-1, 256, 256, 64), (0, 255, 256, 64), (0, 256, 256, 64, 0), (G.num_variants(), 256, 256, 64)):
+        with pytest.raises(G.RidgeGemmError):
+            G.launch_form(*args)
+    assert G.lib().ridge_gemm_launch_form(0, 256, 256, 64, 256, None) == G.HIP_ERROR_INVALID_VALUE
 
 
 @pytest.mark.parametrize("absent", ["_cuda_getDevice", "_cuda_getCurrentRawStream"])
