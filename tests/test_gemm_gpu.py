@@ -37,9 +37,20 @@ def _bits(t):
     return t.cpu().view(torch.int16).numpy().view(np.uint16).ravel()
 
 
-def _run(i, A, B, M, N, K):
+def _cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+def _forms(v, M, N, K):
+    """(label, launch function) of a row's launch and, where that runs smaller blocks than
+    the row's tile, of the row's own tile."""
+    own = [("%s, own tile" % v.label(), G.launch_own_tile)]
+    return [(v.label(), G.launch)] + ([] if G.launch_form(v.index, M, N, K, _cus()).own else own)
+
+
+def _run(i, A, B, M, N, K, launch=G.launch):
     C = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
-    rc = G.launch(i, A, B, C, M, N, K)
+    rc = launch(i, A, B, C, M, N, K)
     assert rc == 0, "variant %d launch returned %d" % (i, rc)
     torch.cuda.synchronize()
     return C
@@ -85,11 +96,12 @@ def test_reference_shapes_all_dividing_variants(M, N, K):
     for v in G.variants():
         if not v.divides(M, N, K):
             continue
-        print("  variant %d %s" % (v.index, v.label()), flush=True)
-        C = _run(v.index, A, B, M, N, K)
-        got = O.f16_bits_to_f32(_bits(C)).reshape(M, N)[rows]
-        ok, frob, mx, ne = O.passes(got, ref, _max_abs(Ab), _max_abs(Bb), K)
-        assert ok, "%s on %dx%dx%d: frob %.3e maxRel %.3e norm %.3e" % (v.label(), M, N, K, frob, mx, ne)
+        for label, launch in _forms(v, M, N, K):
+            print("  variant %d %s" % (v.index, label), flush=True)
+            C = _run(v.index, A, B, M, N, K, launch)
+            got = O.f16_bits_to_f32(_bits(C)).reshape(M, N)[rows]
+            ok, frob, mx, ne = O.passes(got, ref, _max_abs(Ab), _max_abs(Bb), K)
+            assert ok, "%s on %dx%dx%d: frob %.3e maxRel %.3e norm %.3e" % (label, M, N, K, frob, mx, ne)
         tested += 1
     assert tested > 0
 
@@ -115,9 +127,10 @@ def test_small_integer_inputs_bit_exact_every_variant(M, N, K):
     for v in G.variants():
         if not v.divides(M, N, K):
             continue
-        got = _bits(_run(v.index, A, B, M, N, K))
-        bad = int(np.count_nonzero(got != want))
-        assert bad == 0, "%s: %d of %d outputs differ" % (v.label(), bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            got = _bits(_run(v.index, A, B, M, N, K, launch))
+            bad = int(np.count_nonzero(got != want))
+            assert bad == 0, "%s: %d of %d outputs differ" % (label, bad, M * N)
 
 
 @pytest.mark.parametrize("subnormal", ["A", "B", "C"])
@@ -145,9 +158,10 @@ def test_fp16_subnormal_operands_are_not_flushed(subnormal):
     want_bits = want.view(np.uint16).ravel()
     for v in G.variants():
         assert v.divides(M, N, K)
-        got = _bits(_run(v.index, A, B, M, N, K))
-        bad = int(np.count_nonzero(got != want_bits))
-        assert bad == 0, "%s, subnormal %s: %d of %d outputs differ" % (v.label(), subnormal, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            got = _bits(_run(v.index, A, B, M, N, K, launch))
+            bad = int(np.count_nonzero(got != want_bits))
+            assert bad == 0, "%s, subnormal %s: %d of %d outputs differ" % (label, subnormal, bad, M * N)
 
 
 def test_python_gemm_on_offset_views():
@@ -195,13 +209,14 @@ def test_inf_nan_and_overflow_follow_ieee():
     big = torch.full((M, Kb), 16.0, dtype=torch.float16, device=DEV)
     bigB = torch.full((Kb, N), 16.0, dtype=torch.float16, device=DEV)
     for v in G.variants():
-        got = _bits(_run(v.index, A, B, M, N, K)).view(np.float16).reshape(M, N)
-        nan = np.isnan(want)
-        assert np.array_equal(np.isnan(got), nan), "%s: NaN positions differ" % v.label()
-        assert np.array_equal(got[~nan].view(np.uint16), want[~nan].view(np.uint16)), (
-            "%s: %d finite or infinite outputs differ" % (v.label(), int(np.count_nonzero(got[~nan] != want[~nan]))))
-        over = _bits(_run(v.index, big, bigB, M, N, Kb)).view(np.float16)
-        assert np.all(np.isposinf(over)), "%s: 65536 did not round to +inf" % v.label()
+        for label, launch in _forms(v, M, N, K):
+            got = _bits(_run(v.index, A, B, M, N, K, launch)).view(np.float16).reshape(M, N)
+            nan = np.isnan(want)
+            assert np.array_equal(np.isnan(got), nan), "%s: NaN positions differ" % label
+            assert np.array_equal(got[~nan].view(np.uint16), want[~nan].view(np.uint16)), (
+                "%s: %d finite or infinite outputs differ" % (label, int(np.count_nonzero(got[~nan] != want[~nan]))))
+            over = _bits(_run(v.index, big, bigB, M, N, Kb, launch)).view(np.float16)
+            assert np.all(np.isposinf(over)), "%s: 65536 did not round to +inf" % label
 
 
 @pytest.mark.parametrize("key", [(256, 256, 32, 128, 64, 3, 4), (256, 256, 32, 128, 64, 4, 4)])
@@ -262,9 +277,10 @@ def test_random_divisible_shapes_exact_every_variant(M, N, K):
     rows = [v for v in G.variants() if v.divides(M, N, K)]
     assert len(rows) == G.num_variants()
     for v in rows:
-        got = _bits(_run(v.index, A, B, M, N, K))
-        bad = int(np.count_nonzero(got != want))
-        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            got = _bits(_run(v.index, A, B, M, N, K, launch))
+            bad = int(np.count_nonzero(got != want))
+            assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (label, M, N, K, bad, M * N)
 
 
 # Random-data twin of the test above: 3 shapes by default, RIDGE_RANDOM_UNIFORM_SHAPES=n
@@ -291,13 +307,14 @@ def test_random_divisible_shapes_uniform_inputs_every_variant(M, N, K):
     worst_row = (0.0, 0.0, "")
     for v in G.variants():
         assert v.divides(M, N, K)
-        got = O.f16_bits_to_f32(_bits(_run(v.index, A, B, M, N, K))).reshape(M, N)[rows]
-        ok, frob, mx, ne = O.passes(got, ref, max_a, max_b, K)
-        assert ok, "%s on %dx%dx%d: frob %.3e maxRel %.3e norm %.3e" % (v.label(), M, N, K, frob, mx, ne)
-        ok, frob, worst = O.passes_fp16(got, ref, absprod, K)
-        assert ok, "%s on %dx%dx%d: FP16-output gate frob %.3e, worst element at %.2f of its bound" % (
-            v.label(), M, N, K, frob, worst)
-        worst_row = max(worst_row, (worst, frob, v.label()))
+        for label, launch in _forms(v, M, N, K):
+            got = O.f16_bits_to_f32(_bits(_run(v.index, A, B, M, N, K, launch))).reshape(M, N)[rows]
+            ok, frob, mx, ne = O.passes(got, ref, max_a, max_b, K)
+            assert ok, "%s on %dx%dx%d: frob %.3e maxRel %.3e norm %.3e" % (label, M, N, K, frob, mx, ne)
+            ok, frob, worst = O.passes_fp16(got, ref, absprod, K)
+            assert ok, "%s on %dx%dx%d: FP16-output gate frob %.3e, worst element at %.2f of its bound" % (
+                label, M, N, K, frob, worst)
+            worst_row = max(worst_row, (worst, frob, label))
     print("  uniform %dx%dx%d, %d rows checked: worst element at %.3f of its bound (%s), frob %.3e" % (
         M, N, K, len(rows), worst_row[0], worst_row[2], worst_row[1]), flush=True)
 
@@ -330,8 +347,9 @@ def test_ping_pong_tail_tiles_bit_exact(tiles_m, tiles_n, K):
     for v in G.variants():
         if v.schedule != 1 or not v.divides(M, N, K):
             continue
-        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
-        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K, launch)) != want))
+            assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (label, M, N, K, bad, M * N)
 
 
 @pytest.mark.parametrize("tiles_m", [1, 2, 3, 7, 8, 9, 17, 31])
@@ -344,8 +362,9 @@ def test_launch_order_with_ragged_groups_bit_exact(tiles_m, tiles_n):
     Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + 5 * N)
     A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
     for v in G.variants():
-        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
-        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K, launch)) != want))
+            assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (label, M, N, K, bad, M * N)
 
 
 # Grids around the small-grid rule's edges on 256 CUs for every tile size: as 64 x 64
@@ -359,8 +378,9 @@ def test_small_grids_bit_exact_every_variant(M, N, K):
     for v in G.variants():
         if not v.divides(M, N, K):
             continue
-        bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K)) != want))
-        assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            bad = int(np.count_nonzero(_bits(_run(v.index, A, B, M, N, K, launch)) != want))
+            assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (label, M, N, K, bad, M * N)
 
 
 def _persistent_edge_shapes(v):
@@ -389,9 +409,10 @@ def test_persistent_rows_edge_shapes_bit_exact():
             print("  %s %dx%dx%d" % (v.label(), M, N, K), flush=True)
             Ab, Bb, want = _exact_case(M, N, K, -3, 3, M + 7 * N + 13 * K)
             A, B = _to_dev(Ab.ravel(), (M, K)), _to_dev(Bb.ravel(), (K, N))
-            got = _bits(_run(v.index, A, B, M, N, K))
-            bad = int(np.count_nonzero(got != want))
-            assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (v.label(), M, N, K, bad, M * N)
+            for label, launch in _forms(v, M, N, K):
+                got = _bits(_run(v.index, A, B, M, N, K, launch))
+                bad = int(np.count_nonzero(got != want))
+                assert bad == 0, "%s on %dx%dx%d: %d of %d outputs differ" % (label, M, N, K, bad, M * N)
 
 
 # The launcher admits a shape only while its 32-bit in-kernel byte offsets cannot
@@ -428,10 +449,11 @@ def test_largest_k_the_offset_guard_admits_is_exact():
     print("  K = %d, %d variants" % (K, len(rows)), flush=True)
     A, B, want = _offset_limit_case(M, N, K)
     for v in rows:
-        print("  variant %d %s" % (v.index, v.label()), flush=True)
-        got = _bits(_run(v.index, A, B, M, N, K))
-        bad = int(np.count_nonzero(got != want))
-        assert bad == 0, "%s at K = %d: %d of %d outputs differ" % (v.label(), K, bad, M * N)
+        for label, launch in _forms(v, M, N, K):
+            print("  variant %d %s" % (v.index, label), flush=True)
+            got = _bits(_run(v.index, A, B, M, N, K, launch))
+            bad = int(np.count_nonzero(got != want))
+            assert bad == 0, "%s at K = %d: %d of %d outputs differ" % (label, K, bad, M * N)
     del A, B
     torch.cuda.empty_cache()
 
@@ -745,11 +767,13 @@ def test_registered_sweep_shapes_every_variant(M, N, K):
 
 def test_concurrent_host_threads_launch_persistent_rows():
     """Four host threads, each with its own stream and buffers, launch a persistent
-    row 20 times at once (the first launches fill the per-device grid cache
-    concurrently); every result is the exact product of small integers."""
+    row 20 times at once, on a grid that runs its own tiles: all read the per-device
+    cache of its workgroups (and, when this test runs first, fill it at once). Every
+    result is the exact product of small integers."""
     import threading
     v = [w for w in G.variants() if w.schedule == 2][0]
-    M, N, K = 8 * v.BM, 4 * v.BN, 4 * v.BK
+    M, N, K = 20 * v.BM, 15 * v.BN, 4 * v.BK
+    assert G.launch_form(v.index, M, N, K, _cus()).own
     Ab, Bb, want = _exact_case(M, N, K, -3, 3, 77)
     jobs = []
     for t in range(4):
@@ -777,18 +801,23 @@ def test_concurrent_host_threads_launch_persistent_rows():
         assert np.array_equal(_bits(C), want)
 
 
-def test_launches_replay_from_a_captured_hip_graph():
+# Of each schedule: the row's own tiles; the whole grid in smaller blocks; and for the
+# ping-pong row whole rounds with the last in parts.
+@pytest.mark.parametrize("M,N,K,own", [(4096, 3072, 512, (True, True, True)),
+                                       (1024, 1024, 1024, (False, False, False)),
+                                       (4352, 4096, 512, (True, False, True))])
+def test_launches_replay_from_a_captured_hip_graph(M, N, K, own):
     """The launcher allocates nothing and never synchronises, so a caller can
     capture kernel-table launches into a HIP graph and replay them (the way a
     serving loop removes per-launch host cost). One row of each schedule is
     captured on one stream; three replays, with the inputs refilled eagerly
     between them, must each equal eager launches bit for bit."""
-    M, N, K = 1024, 1024, 1024
     picks = []
     for sched in (0, 1, 2):
         cand = [v for v in G.variants() if v.schedule == sched and v.divides(M, N, K)]
         assert cand, "no row of schedule %d divides %dx%dx%d" % (sched, M, N, K)
         picks.append(cand[0])
+        assert G.launch_form(cand[0].index, M, N, K, _cus()).own == own[sched], cand[0].label()
     A = torch.empty((M, K), dtype=torch.float16, device=DEV)
     B = torch.empty((K, N), dtype=torch.float16, device=DEV)
     G.fill_uniform(A, 5)
