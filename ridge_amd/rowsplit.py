@@ -14,6 +14,12 @@ already carries the launch boundary when the calibration switches launchModel
 on). No counterpart in the reference, whose autotuner (tools/ridge-autotune.py)
 ranks single kernel-table rows only.
 
+The model prices a row's own tile. A launch that runs smaller blocks instead, on a
+small grid or in a last round (ridge_gemm_launch_form), takes less, so the time of a
+plan with such a launch is an upper bound: `rank` marks it and names the blocks, and
+only a measurement can put it behind another plan. (The same model on the blocks
+themselves was 38% off on small grids and 16% on last rounds, and is not used.)
+
 `register` writes the plans a measurement of the split decision times, per shape
 of the given registered sweeps that has at least one split: the row measured
 fastest on it in the given sweep CSVs (the anchor), the model's best single row,
@@ -56,6 +62,20 @@ class Plan(namedtuple("Plan", "M N K body rows tail seconds")):
         b = G.variant(self.body).key()
         t = G.variant(self.tail).key() if self.split else (0,) * 7
         return (self.M, self.N, self.K) + b + (self.rows,) + t
+
+    def blocks(self, num_cus=WHOLE_DEVICE_CUS):
+        """What its launches run that is not the row's own tile, "" if nothing: then the
+        model's time is the plan's, else it is an upper bound."""
+        launches = [(self.body, self.rows)] + ([(self.tail, self.M - self.rows)] if self.split else [])
+        out = []
+        for i, m in launches:
+            f = G.launch_form(i, m, self.N, self.K, num_cus)
+            if not f.own:
+                v = G.variant(i)
+                out.append("%d of %d tiles as %d blocks of %dx%d" % (
+                    (m // v.BM) * (self.N // v.BN) - f.ownTiles, (m // v.BM) * (self.N // v.BN), f.partWorkgroups,
+                    f.partBM, f.partBN))
+        return "; ".join(out)
 
     def label(self):
         body = G.variant(self.body).label()
@@ -207,8 +227,18 @@ def _print_rank(ranker, M, N, K, top):
     plans = ranker.rank(M, N, K)
     print("%dx%dx%d: %d single rows, %d split plans" % (M, N, K, sum(not p.split for p in plans),
                                                          sum(p.split for p in plans)))
-    for p in plans[:top]:
-        print("  %9.1f TFLOP/s  %8.2f us  %s" % (2.0 * M * N * K / p.seconds / 1e12, p.seconds * 1e6, p.label()))
+    blocks = [p.blocks(ranker.num_cus) for p in plans]
+    for p, b in list(zip(plans, blocks))[:top]:
+        print(" %s%9.1f TFLOP/s  %s%8.2f us  %s%s" % (">=" if b else "  ", 2.0 * M * N * K / p.seconds / 1e12,
+                                                      "<=" if b else "  ", p.seconds * 1e6, p.label(),
+                                                      " (%s)" % b if b else ""))
+    # A split is only worth offering if no row alone may be as fast: name the rows
+    # whose price is a bound, however far down they stand.
+    rest = [(p, b) for p, b in list(zip(plans, blocks))[top:] if b and not p.split]
+    if rest:
+        print("  further single rows that run smaller blocks than their tile (measure them beside the first):")
+        for p, b in rest:
+            print("    <=%8.2f us  %s (%s)" % (p.seconds * 1e6, p.label(), b))
 
 
 def _print_score(rows):

@@ -49,6 +49,27 @@ def test_a_split_is_priced_as_its_two_launches(ranker):
                    for p in ranker.rank(4096, 4096, 4096))
 
 
+def test_rank_marks_the_plans_whose_launches_run_smaller_blocks(ranker, capsys):
+    """6144 x 3072 x 6144: the model's first plan is a split whose two launches run their
+    own tiles, so its time stands; the same body row alone runs its last 32 of 288 tiles
+    as 256 blocks, and its time, a whole tile more, is only a bound (it measures less
+    than the split)."""
+    plans = ranker.rank(6144, 3072, 6144)
+    assert plans[0].split and plans[0].blocks() == ""
+    alone = next(p for p in plans if not p.split and G.variant(p.body).key() == S3)
+    assert alone.blocks() == "32 of 288 tiles as 256 blocks of 64x128"
+    assert R.main(["rank", "--shape", "6144,3072,6144", "--top", "3"]) == 0
+    out = capsys.readouterr().out
+    first = next(line for line in out.splitlines() if "TFLOP/s" in line)
+    assert "<=" not in first
+    marked = [line for line in out.splitlines() if G.variant(alone.body).label() + " (32 of 288" in line]
+    assert len(marked) == 1 and "<=%8.2f us" % (alone.seconds * 1e6) in marked[0]
+    # A small grid: every row but the 64 x 64 ones runs blocks.
+    assert R.main(["rank", "--shape", "1024,1024,1024", "--top", "24"]) == 0
+    lines = [line for line in capsys.readouterr().out.splitlines() if "TFLOP/s" in line]
+    assert len(lines) == 24 and sum("<=" not in line for line in lines) == 2
+
+
 def test_distinct_splits_keep_one_body_per_split_point_and_tail(ranker):
     got = R.distinct_splits(ranker, 6144, 3072, 6144, 5)
     assert len(got) == 5
