@@ -21,7 +21,9 @@ exists (the reference's own discipline, run-ncu-validation.sh:1-6).
 `run` must be the program rocprofv3 starts (`rocprofv3 ... -- python3 -m
 ridge_amd.labelcheck run`). It launches, for every config in order, the
 registered variant LAUNCHES times on seeded U[-1,1) inputs (and, for a
-registration with a long factor F, LAUNCHES more times at K x F); `gather`
+registration with a long factor F, LAUNCHES more times at K x F), in the row's own
+tile, which is what the model labels, also where ridge_gemm_launch would run smaller
+blocks; `gather`
 assigns the GEMM dispatches of each rocprofv3 pass to configs by dispatch order
 and checks every dispatch's kernel name against the config's template arguments.
 """
@@ -373,7 +375,7 @@ def load_configs(path=CONFIGS_CSV):
 def cmd_run(args):
     """The launches rocprofv3 observes: per config and per K multiplier of its
     registration (`Registration.factors`, the multiplier 1 first), LAUNCHES
-    launches of the registered variant at that K, each followed by a
+    launches of the registered variant in its own tile at that K, each followed by a
     synchronize."""
     import torch
     from ridge_amd import gemm as G
@@ -400,7 +402,7 @@ def cmd_run(args):
             G.fill_uniform(B, 2)
             torch.cuda.synchronize()
             for _ in range(args.launches):
-                rc = G.launch(idx, A, B, C, M, N, K)
+                rc = G.launch_own_tile(idx, A, B, C, M, N, K)
                 if rc != 0:
                     raise SystemExit("config %d: launch returned %d" % (i, rc))
                 torch.cuda.synchronize()

@@ -397,3 +397,27 @@ def test_in_sample_relabelling_figures():
         assert (agree, need) == (55, None)
     results, agree, _, _ = LC.relabel_in_sample(LC._read_rows(REG3.counters), current)
     assert agree == 22 and sum(r["predicted_label"] != "CONTROL" for r, d, lab in results) == 26
+
+
+def test_run_launches_every_config_in_its_own_tile(monkeypatch, tmp_path):
+    """A small grid, and a BK = 32 row that K / 2 takes off the smaller blocks' 64: both
+    durations of a config have to come from the row's own kernel."""
+    torch = pytest.importorskip("torch")
+    from ridge_amd import gemm as G
+    reg = LC.REGISTRATIONS[4]
+    configs = tmp_path / "configs.csv"
+    head = open(reg.configs).read().splitlines()
+    cols = next(line for line in head if not line.startswith("#"))
+    first = dict(zip(cols.split(","), next(line for line in head[head.index(cols) + 1:]).split(",")))
+    first.update(M="512", N="512", K="192", BM="256", BN="256", BK="32", WM="128", WN="64", stages="3", groupM="4")
+    configs.write_text(cols + "\n" + ",".join(first[c] for c in cols.split(",")) + "\n")
+    calls = []
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: None)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    monkeypatch.setattr(G, "fill_uniform", lambda *a: None)
+    monkeypatch.setattr(G, "launch", lambda *a: pytest.fail("not the row's own tile"))
+    monkeypatch.setattr(G, "launch_own_tile", lambda i, A, B, C, M, N, K: calls.append((i, M, N, K)) or 0,
+                        raising=False)
+    assert LC.main(["--registration", "4", "run", "--configs", str(configs)]) in (0, None)
+    i = G.find_variant(256, 256, 32, 128, 64, 3, 4)
+    assert calls == [(i, 512, 512, 192)] * LC.LAUNCHES + [(i, 512, 512, 96)] * LC.LAUNCHES
