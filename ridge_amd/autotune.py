@@ -29,6 +29,7 @@ import tempfile
 from ridge_amd import model as RM
 from ridge_amd import stats as S
 from ridge_amd import tables as T
+from ridge_amd import validate as V
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 DEFAULT_KS = (1, 2, 3, 5, 10, 20)
@@ -143,6 +144,10 @@ def main(argv=None):
     print("  measured sweep   %s" % args.measured)
     print("  hardware model   %s" % hw)
     print("  %d configs over %d shapes (%d per shape)" % (total, nshapes, per_shape))
+    t = T.read(args.measured)
+    blocks = V.in_own_tile(t.records, t.meta).count(False)
+    if blocks:
+        print("  %d of them measured as launched in smaller blocks than their tile, which the model ranks" % blocks)
     print()
     print("  %5s %12s %13s %11s %11s %10s" % ("top_k", "benchmarks", "vs exhaustive", "mean regret",
                                                "max regret", "exact hits"))

@@ -2,7 +2,7 @@
 // registered shape timed on every kernel-table row that divides it.
 //
 //   ridge-measure [sweep.csv] [out.csv] [--allow-skip] [--allow-partitioned]
-//                 [--warmup-seconds S] [--settle-seconds T]
+//                 [--warmup-seconds S] [--settle-seconds T] [--own-tile]
 //   ridge-measure --plans plans.csv out.csv [...]
 //
 // Counterpart of the reference's bench/measure.cu:154-303. Its discipline is
@@ -19,6 +19,13 @@
 // and follow the power the current work draws, so an unsettled measurement
 // partly runs at the previous workload's clock (unsettled 4096^3 canaries
 // spread 6.1% over one sweep, with no trend).
+//
+// --own-tile: every row runs its own tile on every shape
+// (ridge_gemm_launch_own_tile), which is what the cost model predicts and what the
+// committed sweeps measured; for sweeps that score the model. Without it a row is
+// timed as ridge_gemm_launch runs it, on small grids and in last rounds in smaller
+// blocks; for choosing a row. The header's `launch` line says which, and the accuracy
+// report leaves out the rows of an as-launched sweep that ran smaller blocks.
 //
 // --allow-skip: rows of the table that do not divide a shape are recorded as
 // skipped instead of failing the run (for shapes such as N = 128).
@@ -64,6 +71,7 @@ struct Settings {
     bool plans = false;
     bool allowSkip = false;
     bool allowPartitioned = false;
+    bool ownTile = false;
     double warmSeconds = 5.0;
     double settleSeconds = 0.2;
 };
@@ -80,6 +88,8 @@ bool parseSettings(int argc, char** argv, Settings& s) {
             s.plans = true;
         } else if (a == "--allow-partitioned") {
             s.allowPartitioned = true;
+        } else if (a == "--own-tile") {
+            s.ownTile = true;
         } else if (seconds) {
             if (i + 1 >= argc || !ridgeio::toReal(argv[i + 1], *seconds) || *seconds < 0.0) {
                 std::fprintf(stderr, "ridge-measure: %s needs a number of seconds\n", a.c_str());
@@ -95,6 +105,10 @@ bool parseSettings(int argc, char** argv, Settings& s) {
             std::fprintf(stderr, "ridge-measure: unexpected argument %s\n", a.c_str());
             return false;
         }
+    }
+    if (s.plans && s.ownTile) {
+        std::fprintf(stderr, "ridge-measure: --plans times launches as they run, not --own-tile\n");
+        return false;
     }
     return true;
 }
@@ -294,6 +308,7 @@ int main(int argc, char** argv) {
          << "# inputs,U[-1;1) fp16 splitmix64 seeds 1 and 2\n"
          << "# warmup_seconds," << cfg.warmSeconds << "\n"
          << "# settle_seconds," << cfg.settleSeconds << "\n"
+         << "# launch," << (cfg.ownTile ? "own tile" : "as launched") << "\n"
          << "# canary_start_tflops," << canary.first() << "\n";
     if (cfg.plans)
         head << "M,N,K,tag,BM,BN,BK,WM,WN,stages,groupM,body_rows,tail_BM,tail_BN,tail_BK,tail_WM,tail_WN,"
@@ -361,7 +376,9 @@ int main(int argc, char** argv) {
                 ++tally.skipped;
                 continue;
             }
-            auto launch = [&] { return ridge_gemm_launch(v, dA, dB, dC, M, N, K, nullptr); };
+            auto launch = [&] {
+                return (cfg.ownTile ? ridge_gemm_launch_own_tile : ridge_gemm_launch)(v, dA, dB, dC, M, N, K, nullptr);
+            };
             const int rc = launch();
             const hipError_t sync = hipDeviceSynchronize();
             if (rc != 0 || sync != hipSuccess) {

@@ -49,6 +49,21 @@ def registered_gate(records, shapes, keys):
     return want - have, have - want
 
 
+def in_own_tile(records, meta):
+    """One bool per record: the model describes what was timed. All of them in a sweep
+    measured with --own-tile or before launches ran anything else (no `launch` line);
+    in one measured as launched, the rows whose launch runs their own tile throughout."""
+    if meta.get("launch") != "as launched":
+        return [True] * len(records)
+    from ridge_amd import gemm as G
+    cus = int(meta["cus"])
+    out = []
+    for r in records:
+        i = G.find_variant(*(int(r[c]) for c in KEY_COLUMNS))
+        out.append(i < 0 or G.launch_form(i, int(r["M"]), int(r["N"]), int(r["K"]), cus).own)
+    return out
+
+
 @dataclass
 class Joined:
     """One measured row with the model's prediction for it."""
@@ -322,6 +337,14 @@ def main(argv=None):
             else:
                 gate_lines.append("  the measured rows are exactly the registered cross product")
             gate_lines.append("")
+        own = in_own_tile([j.record for j in rows], meta)
+        if not all(own):
+            gate_lines += ["%d of %d rows ran smaller blocks than their tile and are left out: the model describes "
+                           "the tile" % (len(own) - sum(own), len(own)),
+                           "  (ridge-measure --own-tile times every row in its own tile)", ""]
+            rows = [j for j, o in zip(rows, own) if o]
+            if not rows:
+                raise T.TableError(args.measured, 0, "no row ran its own tile: measure with --own-tile")
     except (T.TableError, RuntimeError) as e:
         sys.exit(str(e))
     failed += report(rows, meta, args.hw, gate_lines, args.max_mape, args.fail_mape)

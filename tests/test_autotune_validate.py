@@ -277,3 +277,37 @@ def test_groupm_predictions_tie_exactly_at_equal_footprints(name, concordant, or
         s = tuple(j.record[c] for c in ("M", "N", "K"))
         best[s] = max(best.get(s, 0.0), j.measured)
     assert not [d for d in lo.discordant if best[d[0]] in (d[1][3], d[2][3])]
+
+
+def test_rows_that_ran_smaller_blocks_are_not_held_against_the_model(tmp_path, capsys):
+    """The committed sweep as if it had been measured as launched: the report leaves out
+    the rows whose launch would not run their own tile throughout, the pruner counts
+    them, and a sweep with --own-tile (or with no `launch` line) keeps every row."""
+    path = os.path.join(ROOT, "data", "measured", "mi355x.csv")
+    text = open(path).read()
+    t = T.read(path)
+    assert V.in_own_tile(t.records, t.meta) == [True] * 336
+    sweep = tmp_path / "sweep.csv"
+    sweep.write_text("# launch,own tile\n" + text)
+    t = T.read(str(sweep))
+    assert V.in_own_tile(t.records, t.meta) == [True] * 336
+    sweep.write_text("# launch,as launched\n" + text)
+    t = T.read(str(sweep))
+    own = V.in_own_tile(t.records, t.meta)
+    for r, o in zip(t.records, own):
+        M, N, K = (int(r[c]) for c in ("M", "N", "K"))
+        tiles = (M // int(r["BM"])) * (N // int(r["BN"]))
+        last = tiles % 256
+        if r["schedule"] == "1":
+            assert o == (last == 0 or last > 128), r
+        elif tiles > 128 or (r["BM"], r["BN"]) == ("64", "64"):
+            assert o, r
+        elif tiles <= 64:
+            assert not o, r
+    left = 336 - sum(own)
+    assert 0 < left < 336
+    V.main(["--measured", str(sweep), "--max-mape", "100", "--fail-mape", "100"])
+    out = capsys.readouterr().out
+    assert "%d of 336 rows ran smaller blocks" % left in out and "absolute error (%d rows)" % (336 - left) in out
+    AT.main(["--measured", str(sweep)])
+    assert "%d of them measured as launched in smaller blocks" % left in capsys.readouterr().out

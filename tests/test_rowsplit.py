@@ -165,6 +165,12 @@ def test_ridge_measure_refuses_a_bad_plan_before_touching_the_device(tmp_path, r
     assert not (tmp_path / "out.csv").exists()
 
 
+def test_ridge_measure_refuses_own_tile_with_plans(tmp_path):
+    proc = subprocess.run([MEASURE, "--plans", "plans.csv", str(tmp_path / "out.csv"), "--own-tile"],
+                          capture_output=True, text=True, timeout=60)
+    assert proc.returncode == 2 and "--own-tile" in proc.stderr
+
+
 def test_ridge_measure_refuses_a_plan_list_without_a_column(tmp_path):
     plans = tmp_path / "plans.csv"
     plans.write_text(PLAN_HEADER.replace(",body_rows", "") + "1,1,1,x,1,1,1,1,1,1,1,0,0,0,0,0,0,0\n")

@@ -54,6 +54,29 @@ def test_ridge_measure_writes_the_registered_columns(tmp_path):
 
 
 @pytest.mark.gpu
+def test_ridge_measure_own_tile_times_the_rows_tile(tmp_path):
+    """1024 x 1024 x 2048 as launched and with --own-tile: the 256x256 rows, 16 tiles on
+    256 CUs, run as 64x64 blocks in the one (about 9 us) and in their own tile in the
+    other (over 30), and each file says which."""
+    sweep = tmp_path / "sweep.csv"
+    sweep.write_text("1024,1024,2048,t,\n")
+    ms = {}
+    for flag in ([], ["--own-tile"]):
+        out = tmp_path / "measured.csv"
+        print("step: ridge-measure %s" % flag, flush=True)
+        proc = subprocess.run([os.path.join(BIN, "ridge-measure"), str(sweep), str(out), "--warmup-seconds", "1",
+                               "--settle-seconds", "0.05"] + flag, cwd=ROOT, capture_output=True, text=True,
+                              timeout=300)
+        assert proc.returncode == 0, proc.stdout[-4000:] + proc.stderr[-2000:]
+        lines = out.read_text().splitlines()
+        assert ("# launch,own tile" if flag else "# launch,as launched") in lines
+        rows = list(csv.DictReader(line for line in lines if not line.startswith("#")))
+        ms[bool(flag)] = [float(r["ms"]) for r in rows if (r["BM"], r["BN"]) == ("256", "256")]
+    assert len(ms[True]) == len(ms[False]) == 10
+    assert all(own > 2 * launched for own, launched in zip(ms[True], ms[False])), ms
+
+
+@pytest.mark.gpu
 def test_ridge_measure_times_registered_launch_plans(tmp_path):
     """--plans: one single-row plan and one row split of 1536 x 1536 x 512 (the
     64x64 row on 1024 rows, the 128x128 persistent row on the other 512; any
