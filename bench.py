@@ -35,7 +35,9 @@ work), reported in TFLOP/s with the thread count used (the cores this process ma
 run on, at most 16).
 
 model: the calibrated cost model's prediction for the measured variant and shape
-(TFLOP/s, label, error against `value`), read from data/hardware/mi355x.json.
+(TFLOP/s, label, error against `value`), read from data/hardware/mi355x.json. It
+describes the row's own tile; where the launch runs smaller blocks, on a small grid or
+in a last round, `smaller_blocks` says which, and the figure is not of what was timed.
 
 --split-tail: a step is a row split instead, two launches on one stream: --variant
 on the first R rows of C (by default the rows of whole rounds of its resident
@@ -334,6 +336,14 @@ def autotune_regret(k=10):
         return {"error": "%s" % e}
 
 
+def smaller_blocks(body, M, N, K, tail=None, rows=None):
+    """{"smaller_blocks": text} for launches that run smaller blocks than their row's
+    tile, which the model does not describe; {} for the others."""
+    from ridge_amd import rowsplit as R
+    text = R.Plan(M, N, K, body.index, rows or M, tail.index if tail else None, 0.0).blocks()
+    return {"smaller_blocks": text} if text else {}
+
+
 def model_prediction(v, M, N, K, measured):
     """The calibrated cost model's prediction for the variant this run measured:
     TFLOP/s, bottleneck label and the error against the measurement."""
@@ -346,7 +356,7 @@ def model_prediction(v, M, N, K, measured):
         return {"error": "%s" % e}
     return {"predicted_tflops": round(p["predictedTFLOPS"], 1), "label": p["bottleneck"],
             "error_pct": round((p["predictedTFLOPS"] - measured) / measured * 100, 1),
-            "hardware": os.path.relpath(HARDWARE_JSON, ROOT)}
+            "hardware": os.path.relpath(HARDWARE_JSON, ROOT), **smaller_blocks(v, M, N, K)}
 
 
 def model_split_prediction(body, tail, rows, M, N, K, measured):
@@ -367,7 +377,7 @@ def model_split_prediction(body, tail, rows, M, N, K, measured):
     tflops = 2.0 * M * N * K / secs / 1e12
     return {"predicted_tflops": round(tflops, 1), "label": "+".join(labels),
             "error_pct": round((tflops - measured) / measured * 100, 1),
-            "hardware": os.path.relpath(HARDWARE_JSON, ROOT)}
+            "hardware": os.path.relpath(HARDWARE_JSON, ROOT), **smaller_blocks(body, M, N, K, tail, rows)}
 
 
 def cpu_baseline(M, N, K, seconds=10.0):

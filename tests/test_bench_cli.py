@@ -24,3 +24,18 @@ def test_window_statistics():
     s = bench.window_summary(flops, [1.0, 2.0, 1.25, 1.0, 4.0])
     assert s["tflops"] == 1600.0 and s["max"] == 2000.0 and s["min"] == 500.0 and s["windows"] == 5
     assert s["range_pct"] == 93.75
+
+
+def test_model_figure_says_where_the_launch_runs_smaller_blocks():
+    """The headline launch runs its own tile; 6144 x 3072 x 6144 on the same row has a
+    last round in blocks, its split has none, and 1024 cubed is all blocks."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from ridge_amd import gemm as G
+    v = G.variant(G.find_variant(*bench.DEFAULT_VARIANT))
+    tail = G.variant(G.find_variant(128, 128, 64, 64, 64, 4, 8))
+    assert "smaller_blocks" not in bench.model_prediction(v, *bench.DEFAULT_SHAPE, 1400.0)
+    got = bench.model_prediction(v, 6144, 3072, 6144, 1200.0)
+    assert got["smaller_blocks"] == "32 of 288 tiles as 256 blocks of 64x128"
+    assert "smaller_blocks" not in bench.model_split_prediction(v, tail, 5376, 6144, 3072, 6144, 1200.0)
+    assert bench.model_prediction(v, 1024, 1024, 1024, 300.0)["smaller_blocks"].startswith("16 of 16 tiles")
