@@ -208,7 +208,11 @@ int tailParts(int rem, int slots, int N, int K, int most) {
 // 6400 x 768 88.3 -> 86.0, 93.0 -> 85.2; 15104 x 15104 x 512 219.5 -> 216.5, 232.9 ->
 // 224.4; 256x128x64 s3 at 8192 x 4096 x 512 41.6 -> 39.8, 49.8 -> 46.6. Two rounds
 // gained up to 20% on one device and lost up to 2% on another (8192 x 4096 x 512 40.2
-// -> 36.9, 34.8 -> 34.9; 6144 x 6144 x 512 41.5 -> 42.3).
+// -> 36.9, 34.8 -> 34.9; 6144 x 6144 x 512 41.5 -> 42.3). The shortest K loops gain the
+// most, the mean of the eight 256x256x32 rows: 8192 x 8192 x 32 29.3 -> 24.7, x 64 33.9
+// -> 30.8, x 128 39.6 -> 34.5, x 192 47.2 -> 44.0; 12288 x 4096 (three rounds) x 32 21.9
+// -> 19.7, x 64 24.3 -> 21.2; the least 8192 x 6144 x 32 21.3 -> 19.1, x 64 24.2 -> 24.7
+// (four of the rows 2-8% slower), x 96 25.7 -> 25.0, x 128 27.5 -> 25.5.
 int phaseWidth(int wholeTiles, int slots, int K) {
     return slots >= ridge::kPhases && wholeTiles / slots >= 3 && K <= 2048 ? slots / ridge::kPhases : 0;
 }
