@@ -48,9 +48,10 @@ figure is the sum of the two predicted launch times; `roofline.traffic` is null
 (no profile covers a pair of launches).
 
 autotune: the metric's second half, the mean top-10 regret of the model-pruned
-autotuner, is computed from the committed measured sweep of the current kernels
-(data/measured/mi355x-current-kernels.csv, 14 shapes x 24 variants; the same sweep with
-the previous kernels, data/measured/mi355x.csv, beside it) and the committed
+autotuner, is computed from the committed measured sweep of the rows' own tiles
+(data/measured/mi355x-current-kernels.csv, 14 shapes x 24 variants, taken before launches
+ran any smaller blocks; the same sweep with the kernels before the steady K-loop
+passes, data/measured/mi355x.csv, beside it) and the committed
 calibration (data/hardware/mi355x.json)
 by ridge_amd.autotune, with regret at top-1 and the expected regret of a random
 shortlist beside it, and the same for the twelve held-out sweeps, each registered
@@ -76,9 +77,10 @@ DEFAULT_SHAPE = (4096, 4096, 4096)
 # measurement, data/measured/mi355x-baseline-configs.csv).
 DEFAULT_VARIANT = (256, 256, 32, 128, 64, 3, 4)
 PROFILES = os.path.join(ROOT, "profiles")
-# The in-sample sweep measured with the current kernels, and the same sweep with
-# the kernels before the steady K-loop passes (the set every earlier figure and
-# the held-out comparisons refer to).
+# The in-sample sweep of the rows' own tiles, with the steady K-loop passes and the K
+# stagger and before launches ran smaller blocks, and the same sweep with the kernels
+# before the steady passes (the set every earlier figure and the held-out comparisons
+# refer to).
 MEASURED_SWEEP = os.path.join(ROOT, "data", "measured", "mi355x-current-kernels.csv")
 MEASURED_SWEEP_PREVIOUS = os.path.join(ROOT, "data", "measured", "mi355x.csv")
 HARDWARE_JSON = os.path.join(ROOT, "data", "hardware", "mi355x.json")
@@ -290,9 +292,9 @@ def measured_traffic(M, N, K, key, cold=False):
 
 def autotune_regret(k=10):
     """The pruner's regret at top-1 and top-k with the random-shortlist baseline,
-    on the committed in-sample sweep measured with the current kernels
+    on the committed in-sample sweep of the rows' own tiles
     (data/measured/mi355x-current-kernels.csv, 14 shapes x 24 variants, current
-    calibration), on the same sweep with the previous kernels
+    calibration), on the same sweep with the kernels before the steady K-loop passes
     (data/measured/mi355x.csv) and on the twelve held-out sweeps, each
     registered before it was measured and scored with the constants frozen with
     it (data/measured/mi355x-heldout*.csv); a property of the
