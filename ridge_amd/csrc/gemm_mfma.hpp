@@ -375,6 +375,11 @@ __device__ __forceinline__ void storeStaged(const float4_t (&acc)[TM][TN], RIDGE
 // 17.3 against 17.2 | 18.5 against 17.2. Non-temporal, rows lost up to 12% to the cached
 // stores of a kernel without the phased start; cached, none does. At K = 64 eight Cs in
 // turn are 3-12% faster non-temporal and one C between 10% faster and 9% slower.
+// From K = 64 the mean over shapes of 64 MiB to 256 MiB and K to 320 is for every row at
+// least as fast as without (one C up to 13% faster and 1% slower, Cs in turn 4-15%
+// faster); the worst single cases rewrite one C whose rows are a power of two apart:
+// 256x256x64 w64x128 at 8192 x 8192 x 128 40.2 -> 43.7 us (Cs in turn 44.4 -> 43.5) and x
+// 1024 122.4 -> 127.7 (123.7 -> 128.5).
 constexpr size_t kNonTemporalBytes = (size_t)64 << 20;
 constexpr int kNonTemporalPingPongK = 64;
 
